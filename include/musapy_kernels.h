@@ -330,6 +330,8 @@ int musapy_binary_mixed_v2(int op, const void* a, int a_dtype, const void* b, in
  *  - SUM, PROD and MEAN along a strided axis whose outputs are unit-stride (column reductions):
  *    the column kernel's (column group, tile) blocks publish their per-column results and count
  *    themselves per group; the block that completes a group's count folds its tiles in order.
+ *  - narrow rows of a strided axis, and strided axes with many outputs, for every op: one launch,
+ *    or a second one that folds the tiles' partials (kept in `workspace`, as many tiles as fit).
  * Either way the result is independent of block timing.  `c` receives the values (the int64
  * indices for ARGMAX/ARGMIN); `dtype` is the compute dtype (F32, F64 or I64 for every op; C64 and
  * C128 for SUM, PROD and MEAN; MEAN takes a floating or complex dtype).  The payload of

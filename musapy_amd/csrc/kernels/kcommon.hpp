@@ -103,6 +103,31 @@ __device__ inline Vec<T, N> vload_nt(const T* p) {
   __builtin_memcpy(&v, w, sizeof(v));
   return v;
 }
+// Vectors at any element address: N consecutive elements from a pointer that is aligned to the
+// element only (a row of odd length, a slice that starts anywhere).  Global memory accepts 16-byte
+// accesses at 4-byte (and, in the unaligned access mode that HIP programs run in, any) addresses, so
+// these compile to the same global_load_dwordx4 as the aligned forms; a wave's 1 KB run that starts
+// inside a cache line only touches one line more.
+template <int B, int A> struct ElWord {
+  typedef typename NtWord<B>::type type __attribute__((aligned(A)));
+};
+template <typename T, int N>
+__device__ inline Vec<T, N> vload_el(const T* p, bool nt) {
+  constexpr int kB = int(sizeof(T) * N);
+  constexpr int kW = kB > 16 ? 16 : kB;
+  constexpr int kA = int(alignof(T)) < kW ? int(alignof(T)) : kW;
+  using W = typename NtWord<kW>::type;
+  using U = typename ElWord<kW, kA>::type;
+  static_assert(sizeof(W) == kW && kB % kW == 0, "element-aligned load width");
+  W w[kB / kW];
+#pragma unroll
+  for (int i = 0; i < kB / kW; ++i)
+    w[i] = nt ? __builtin_nontemporal_load(reinterpret_cast<const U*>(p) + i) : reinterpret_cast<const U*>(p)[i];
+  Vec<T, N> v;
+  __builtin_memcpy(&v, w, kB);
+  return v;
+}
+
 template <typename T, int N>
 __device__ inline void vstore_nt(T* p, const Vec<T, N>& v) {
   constexpr int kB = int(sizeof(Vec<T, N>));

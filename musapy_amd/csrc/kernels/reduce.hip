@@ -8,7 +8,9 @@
 //        when the axis is unit-stride, then combines through wave-64 butterflies and LDS;
 //   col  the reduced axis is strided but the innermost output dim is unit-stride (axis=0 of a
 //        C-order matrix): 64 lanes x VEC walk adjacent columns, the 4 waves of a block split the
-//        rows, and LDS merges the waves -- every load is a coalesced row segment.
+//        rows, and LDS merges the waves -- every load is a coalesced row segment.  Narrow rows
+//        take whole rows per step instead (span kernel), and reductions with many outputs one
+//        lane per 16 bytes of them (lane kernel); col_route holds the lines between the three.
 // Large reductions are split into tiles: the partial entry points write [out_size][tiles] and
 // the final entry points reduce those rows with the same row kernel.  Every combine order is
 // fixed, so results are identical from run to run.
@@ -656,20 +658,28 @@ struct ColArgs {
   bool nt;            // streaming loads
 };
 
+// A lane's first column.  The last vector of a row of odd length is moved back to end with the row
+// (the columns it shares with its neighbour are reduced twice, with the same result).
+template <int VEC>
+__device__ inline uint64_t lane_col(const ColArgs& ca, uint32_t cg, int lane) {
+  const uint64_t c0 = (uint64_t(cg) * kWave + uint64_t(lane)) * VEC;
+  return c0 < ca.C && c0 + VEC > ca.C && ca.C >= VEC ? ca.C - VEC : c0;
+}
+
 // One (column group, tile) block of a column reduction: lane `lane` of wave 0 ends with the
 // block's accumulators r[v] of its VEC columns (indices relative to the tile) and first[v], the
 // elements of axis row 0 when the tile starts there.  `part` is the block's LDS for the waves.
 template <class Op, class T, int VEC, int UNROLL, int BS = kRBlock>
-__device__ inline void col_partial(const T* __restrict__ a, const ColArgs& ca, bool vec_ok, uint32_t t, uint32_t cg,
+__device__ inline void col_partial(const T* __restrict__ a, const ColArgs& ca, uint32_t t, uint32_t cg,
                                    uint32_t outer, typename Op::A (&part)[BS / kWave - 1][kWave * VEC],
                                    typename Op::A (&acc)[VEC], T (&first)[VEC]) {
   constexpr int kWaves = BS / kWave;
   const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
   int64_t off[1];
   row_offsets<1>(ca.ix, outer, off);
-  const uint64_t c0 = uint64_t(cg) * kWave * VEC + uint64_t(lane) * VEC;
+  const uint64_t c0 = lane_col<VEC>(ca, cg, lane);
   const T* base = a + off[0] + c0;
-  const bool full = vec_ok && c0 + VEC <= ca.C;
+  const bool full = c0 + VEC <= ca.C;
   const uint64_t k0 = uint64_t(t) * ca.chunk;
   const uint64_t k1 = k0 + ca.chunk < ca.R ? k0 + ca.chunk : ca.R;
 #pragma unroll
@@ -683,7 +693,7 @@ __device__ inline void col_partial(const T* __restrict__ a, const ColArgs& ca, b
       // the axis's row 0 for the NaN-at-0 rule: one extra load by wave 0 of tile 0, kept out of
       // the streaming loop (a capture inside it cost the ordered kernels ~10% on (8192, 8192))
       if (Op::kOrdered && k == 0 && k < k1) {
-        const Vec<T, VEC> x = vload_pol<T, VEC>(base, ca.nt);
+        const Vec<T, VEC> x = vload_el<T, VEC>(base, ca.nt);
 #pragma unroll
         for (int v = 0; v < VEC; ++v) first[v] = x.v[v];
       }
@@ -698,7 +708,7 @@ __device__ inline void col_partial(const T* __restrict__ a, const ColArgs& ca, b
       Vec<T, VEC> x[UNROLL], y[UNROLL];  // ping-pong buffers
       auto load = [&](uint64_t kk, Vec<T, VEC>(&d)[UNROLL]) {
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u) d[u] = vload_pol<T, VEC>(base + int64_t(kk + u * kWaves) * ca.rs, ca.nt);
+        for (int u = 0; u < UNROLL; ++u) d[u] = vload_el<T, VEC>(base + int64_t(kk + u * kWaves) * ca.rs, ca.nt);
       };
       auto fold = [&](uint64_t kk, const Vec<T, VEC>(&src)[UNROLL]) {
 #pragma unroll
@@ -736,7 +746,7 @@ __device__ inline void col_partial(const T* __restrict__ a, const ColArgs& ca, b
         }
       }
       for (; k < k1; k += kWaves) {
-        Vec<T, VEC> x = vload_pol<T, VEC>(base + int64_t(k) * ca.rs, ca.nt);
+        Vec<T, VEC> x = vload_el<T, VEC>(base + int64_t(k) * ca.rs, ca.nt);
 #pragma unroll
         for (int v = 0; v < VEC; ++v) acc[v] = Op::step(acc[v], x.v[v], int64_t(k - k0));
       }
@@ -765,7 +775,7 @@ __device__ inline void col_partial(const T* __restrict__ a, const ColArgs& ca, b
 }
 
 template <class Op, class T, int VEC, int UNROLL, int WRITE, int BS = kRBlock>
-__global__ __launch_bounds__(BS) void k_reduce_col(const T* __restrict__ a, ColArgs ca, RedOut<T> out, bool vec_ok) {
+__global__ __launch_bounds__(BS) void k_reduce_col(const T* __restrict__ a, ColArgs ca, RedOut<T> out) {
   using A = typename Op::A;
   __shared__ A part[BS / kWave - 1][kWave * VEC];
   const uint32_t b = blockIdx.x;
@@ -775,9 +785,9 @@ __global__ __launch_bounds__(BS) void k_reduce_col(const T* __restrict__ a, ColA
   const uint32_t outer = rest / ca.cgroups;
   A acc[VEC];
   T first[VEC];
-  col_partial<Op, T, VEC, UNROLL, BS>(a, ca, vec_ok, t, cg, outer, part, acc, first);
+  col_partial<Op, T, VEC, UNROLL, BS>(a, ca, t, cg, outer, part, acc, first);
   const int lane = threadIdx.x % kWave;
-  const uint64_t c0 = uint64_t(cg) * kWave * VEC + uint64_t(lane) * VEC;
+  const uint64_t c0 = lane_col<VEC>(ca, cg, lane);
   if (threadIdx.x < kWave && c0 < ca.C) {
 #pragma unroll
     for (int v = 0; v < VEC; ++v) {
@@ -791,6 +801,243 @@ __global__ __launch_bounds__(BS) void k_reduce_col(const T* __restrict__ a, ColA
 }
 
 // --------------------------------------------------------------------------------------------
+// span kernel: column reductions of narrow rows.  A block of `bs` lanes reads `lanes` of them
+// (lanes * VEC elements, a whole number m of rows) per step, so every lane keeps the same VEC
+// columns for the whole walk and loads are contiguous over the block whatever the row length: 37
+// columns of f32 take 481 of 512 lanes (13 rows a step), where 64 lanes per row group of the column
+// kernel left 54 of 64 idle.  Rows that are not contiguous, or a strip of wider rows, work the same
+// as long as the strip holds whole vectors.  Tile t of a slice takes chunks t, t + tiles, ... of
+// m * UNROLL rows, so the blocks in flight read neighbouring memory.  The m row residues meet in
+// LDS (a tree over rows: fixed order).  With several tiles the block's accumulators go to `part`
+// ([slice][tile][column]) and k_span_final folds them.
+struct SpanArgs {
+  RowIndexer<1> ix;    // outer output dims -> input offset
+  uint32_t C;          // innermost output extent (unit stride in the input)
+  uint32_t cw;         // columns per strip (== C when one strip)
+  uint32_t strips;
+  uint32_t m, lanes;   // rows and lanes per step
+  uint32_t tiles;
+  uint32_t whole;      // whole chunks (m * UNROLL rows) of a slice
+  uint64_t R;
+  int64_t rs;
+  bool flat;           // rows are contiguous (rs == C, one strip): a vector may run into the next row
+};
+constexpr int kSpanBS = 512;
+constexpr int kSpanUnroll = 8;
+
+template <class Op, class T, int VEC, int UNROLL, bool FINAL>
+__global__ __launch_bounds__(kSpanBS) void k_reduce_span(const T* __restrict__ a, SpanArgs sa, RedOut<T> out,
+                                                         typename Op::A* __restrict__ part) {
+  using A = typename Op::A;
+  __shared__ A s[kSpanBS * VEC];
+  const uint32_t b = blockIdx.x;
+  const uint32_t t = b % sa.tiles;
+  const uint32_t rest = b / sa.tiles;
+  const uint32_t strip = rest % sa.strips;
+  const uint32_t outer = rest / sa.strips;
+  int64_t off[1];
+  row_offsets<1>(sa.ix, outer, off);
+  const uint32_t cbase = strip * sa.cw;
+  const uint32_t l = threadIdx.x;
+  const uint32_t e = l * VEC;           // the lane's first element of a step (row-major over the strip)
+  const uint32_t r0 = e / sa.cw, c0 = e - r0 * sa.cw;
+  const uint32_t width = sa.cw < sa.C - cbase ? sa.cw : sa.C - cbase;  // columns of this strip
+  const bool live = l < sa.lanes && c0 < width;
+  const T* p = a + off[0] + cbase;
+  const uint32_t step_rows = sa.m * UNROLL;
+  A acc[VEC];
+  uint32_t rv[VEC];                     // row of element v inside a step
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) {
+    acc[v] = Op::init();
+    rv[v] = sa.flat ? (e + v) / sa.cw : r0;
+  }
+  if (live) {
+    const T* lp = p + int64_t(r0) * sa.rs + c0;
+    Vec<T, VEC> buf[2][UNROLL];
+    auto load = [&](uint64_t k, Vec<T, VEC>(&d)[UNROLL]) {
+      const T* q = lp + int64_t((uint64_t(t) + k * sa.tiles) * step_rows) * sa.rs;
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) d[u] = vload_el<T, VEC>(q + int64_t(uint64_t(u) * sa.m) * sa.rs, true);
+    };
+    auto fold = [&](uint64_t k, const Vec<T, VEC>(&src)[UNROLL]) {
+      const uint32_t row = uint32_t((uint64_t(t) + k * sa.tiles) * step_rows);
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        T xs[UNROLL][1];
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) xs[u][0] = src[u].v[v];
+        acc[v] = Op::template step_chunk<UNROLL, 1>(acc[v], xs, row + rv[v], sa.m);
+      }
+    };
+    const uint64_t mine = t < sa.whole ? (sa.whole - t - 1) / sa.tiles + 1 : 0;
+    walk_chunks(mine, buf, load, fold, [] {});
+    if (t == sa.whole % sa.tiles && uint64_t(sa.whole) * step_rows < sa.R) {
+      // The rows past the last whole chunk, in one round of unconditional loads (a lane without a
+      // row reads the slice's first elements and drops them): with the loads under a condition the
+      // compiler waits for each before the next, 8 round trips of about 1 us.
+      const uint64_t base = uint64_t(sa.whole) * step_rows;
+      Vec<T, VEC> x[UNROLL];
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        const uint64_t row = base + uint64_t(u) * sa.m;
+        const T* q = row + rv[VEC - 1] < sa.R ? lp + int64_t(row) * sa.rs : p;
+        x[u] = vload_el<T, VEC>(q, true);
+      }
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        const uint64_t row = base + uint64_t(u) * sa.m;
+        if (row + rv[VEC - 1] < sa.R) {
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) acc[v] = Op::step(acc[v], x[u].v[v], int64_t(row + rv[v]));
+        } else if (row + rv[0] < sa.R) {  // the vector that the end of the slice cuts (flat rows)
+          const T* q = lp + int64_t(row) * sa.rs;
+#pragma unroll
+          for (int v = 0; v < VEC; ++v)
+            if (row + rv[v] < sa.R) acc[v] = Op::step(acc[v], q[v], int64_t(row + rv[v]));
+        }
+      }
+    }
+  }
+  // the m x cw accumulators of the block, in row-major order
+  if (l < sa.lanes) {
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) s[e + v] = acc[v];
+  }
+  __syncthreads();
+  for (uint32_t rows = sa.m; rows > 1;) {
+    const uint32_t half = (rows + 1) / 2;
+    const uint32_t n = (rows - half) * sa.cw;
+    for (uint32_t i = l; i < n; i += blockDim.x) s[i] = Op::comb(s[i], s[i + half * sa.cw]);
+    __syncthreads();
+    rows = half;
+  }
+  for (uint32_t i = l; i < width; i += blockDim.x) {
+    A r = s[i];
+    if constexpr (FINAL) {
+      if constexpr (Op::kOrdered) r = absorb_first<Op, T>(r, p[i]);
+      write_result<Op, T, kWriteFinal>(out, uint64_t(outer) * sa.C + cbase + i, r, 0);
+    } else {
+      part[(uint64_t(outer) * sa.tiles + t) * sa.C + cbase + i] = r;
+    }
+  }
+}
+
+// Folds part[slice][tile][column] over the tiles, in order, and returns the words it read to zero
+// (the workspace rule).  A block takes `cb` columns of one slice, kSpanBS / cb lanes per column.
+template <class Op, class T>
+__global__ __launch_bounds__(kSpanBS) void k_span_final(const T* __restrict__ a, typename Op::A* __restrict__ part,
+                                                        RowIndexer<1> ix, uint32_t C, uint32_t tiles, uint32_t cb,
+                                                        uint32_t groups, RedOut<T> out) {
+  using A = typename Op::A;
+  __shared__ A s[kSpanBS];
+  const uint32_t outer = blockIdx.x / groups;
+  const uint32_t g = blockIdx.x - outer * groups;
+  const uint32_t tl = threadIdx.x / cb, c = threadIdx.x - tl * cb;
+  const uint32_t rows = kSpanBS / cb;  // lanes per column
+  const uint32_t col = g * cb + c;
+  const bool live = tl < rows && col < C;
+  A* q = part + uint64_t(outer) * tiles * C + col;
+  A acc = Op::init();
+  if (live) {
+    constexpr int U = 8;
+    uint32_t t = tl;
+    for (; t + (U - 1) * rows < tiles; t += U * rows) {
+      A x[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[u] = q[uint64_t(t + u * rows) * C];
+#pragma unroll
+      for (int u = 0; u < U; ++u) acc = Op::comb(acc, x[u]);
+    }
+    for (; t < tiles; t += rows) acc = Op::comb(acc, q[uint64_t(t) * C]);
+  }
+  if (tl < rows) s[threadIdx.x] = acc;
+  T first{};
+  if constexpr (Op::kOrdered) {
+    if (live && tl == 0) {
+      int64_t off[1];
+      row_offsets<1>(ix, outer, off);
+      first = a[off[0] + col];
+    }
+  }
+  __syncthreads();
+  for (uint32_t n = rows; n > 1;) {
+    const uint32_t half = (n + 1) / 2;
+    if (tl < n - half) s[threadIdx.x] = Op::comb(s[threadIdx.x], s[threadIdx.x + half * cb]);
+    __syncthreads();
+    n = half;
+  }
+  if (live && tl == 0) {
+    A r = s[c];
+    if constexpr (Op::kOrdered) r = absorb_first<Op, T>(r, first);
+    write_result<Op, T, kWriteFinal>(out, uint64_t(outer) * C + col, r, 0);
+  }
+  if (live) {
+    constexpr int W = int(sizeof(A) / 4);
+    for (uint32_t t = tl; t < tiles; t += rows) {
+      uint32_t* w = reinterpret_cast<uint32_t*>(q + uint64_t(t) * C);
+#pragma unroll
+      for (int i = 0; i < W; ++i) w[i] = 0;
+    }
+  }
+}
+
+// lane kernel: column reductions with enough outputs to fill the GPU with one lane per VEC of
+// them.  Each lane walks the whole axis (in the reference's order), 8 rows of loads in flight; no
+// LDS, no second level.  The last vector of a row is moved back to end with the row: its columns
+// are computed twice, with the same result.
+template <class Op, class T, int VEC, int UNROLL>
+__global__ __launch_bounds__(kRBlock) void k_reduce_lane(const T* __restrict__ a, RowIndexer<1> ix, uint32_t C,
+                                                         FastDiv vpr, uint64_t R, int64_t rs, uint32_t items,
+                                                         RedOut<T> out) {
+  using A = typename Op::A;
+  const uint32_t g = blockIdx.x * kRBlock + threadIdx.x;
+  if (g >= items) return;
+  const uint32_t outer = fd_div(vpr, g);
+  uint32_t c0 = (g - outer * vpr.d) * VEC;
+  if (c0 + VEC > C) c0 = C - VEC;
+  int64_t off[1];
+  row_offsets<1>(ix, outer, off);
+  const T* p = a + off[0] + c0;
+  A acc[VEC];
+  T first[VEC];
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) {
+    acc[v] = Op::init();
+    first[v] = T{};
+  }
+  if constexpr (Op::kOrdered) {
+    const Vec<T, VEC> x = vload_el<T, VEC>(p, true);
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) first[v] = x.v[v];
+  }
+  uint64_t k = 0;
+  for (; k + UNROLL <= R; k += UNROLL) {
+    Vec<T, VEC> x[UNROLL];
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) x[u] = vload_el<T, VEC>(p + int64_t(k + u) * rs, true);
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) {
+      T xs[UNROLL][1];
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) xs[u][0] = x[u].v[v];
+      acc[v] = Op::template step_chunk<UNROLL, 1>(acc[v], xs, uint32_t(k), 1);
+    }
+  }
+  for (; k < R; ++k) {
+    const Vec<T, VEC> x = vload_el<T, VEC>(p + int64_t(k) * rs, true);
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) acc[v] = Op::step(acc[v], x.v[v], int64_t(k));
+  }
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) {
+    A r = acc[v];
+    if constexpr (Op::kOrdered) r = absorb_first<Op, T>(r, first[v]);
+    write_result<Op, T, kWriteFinal>(out, uint64_t(outer) * C + c0 + v, r, 0);
+  }
+}
+
+// --------------------------------------------------------------------------------------------
 // Column sums, products and means in one launch: the (column group, tile) blocks of k_reduce_col
 // count themselves in their group's counter as they start and publish wave 0's per-column
 // accumulators (tagged relaxed words, publish.hpp) as they finish; the block whose increment
@@ -800,7 +1047,7 @@ __global__ __launch_bounds__(BS) void k_reduce_col(const T* __restrict__ a, ColA
 // slower than partial + final; counting at the end instead of the start cost 0.35 us more).
 template <class Op, class T, int VEC, int UNROLL, int BS>
 __global__ __launch_bounds__(BS) void k_reduce_col_last(const T* __restrict__ a, ColArgs ca, RedOut<T> out,
-                                                        bool vec_ok, FusedArgs fa, uint32_t* counters) {
+                                                        FusedArgs fa, uint32_t* counters) {
   using A = typename Op::A;
   static_assert(!Op::kOrdered && sizeof(A) % 4 == 0, "value folds of 32-bit slices");
   constexpr int W = int(sizeof(A) / 4);
@@ -817,9 +1064,9 @@ __global__ __launch_bounds__(BS) void k_reduce_col_last(const T* __restrict__ a,
   if (threadIdx.x == 0) arrived = atomicAdd(counters + group, 1u);
   A acc[VEC];
   T first[VEC];
-  col_partial<Op, T, VEC, UNROLL, BS>(a, ca, vec_ok, t, cg, outer, part, acc, first);
+  col_partial<Op, T, VEC, UNROLL, BS>(a, ca, t, cg, outer, part, acc, first);
   const int lane = threadIdx.x % kWave;
-  const uint64_t c0 = uint64_t(cg) * kWave * VEC + uint64_t(lane) * VEC;
+  const uint64_t c0 = lane_col<VEC>(ca, cg, lane);
   auto slot = [&](uint32_t tt, int v) {
     return fa.slots + ((uint64_t(group) * ca.tiles + tt) * (kWave * VEC) + uint64_t(lane) * VEC + v) * W;
   };
@@ -913,7 +1160,7 @@ __global__ __launch_bounds__(BS) void k_reduce_col_last(const T* __restrict__ a,
 // its lanes' columns into one (value, col * R + row) key, skipping columns whose row 0 is NaN,
 // and publishes it; the last block of the grid combines the published keys in a fixed order.
 template <class Op, class OpF, class T, int VEC, int UNROLL, int BS, int PER>
-__global__ __launch_bounds__(BS) void k_reduce_col2d(const T* __restrict__ a, ColArgs ca, uint32_t nblk, bool vec_ok,
+__global__ __launch_bounds__(BS) void k_reduce_col2d(const T* __restrict__ a, ColArgs ca, uint32_t nblk,
                                                      RedOut<T> out, FusedArgs fa) {
   using A = typename Op::A;
   using AF = typename OpF::A;
@@ -927,7 +1174,7 @@ __global__ __launch_bounds__(BS) void k_reduce_col2d(const T* __restrict__ a, Co
     const uint32_t cg = b / ca.tiles;
     // which of wave 0's columns head with a NaN (pass 2 drops them): read before the stream, so
     // the loads overlap it
-    const uint64_t c0 = uint64_t(cg) * kWave * VEC + uint64_t(threadIdx.x % kWave) * VEC;
+    const uint64_t c0 = lane_col<VEC>(ca, cg, threadIdx.x % kWave);
     uint32_t nan_head = 0;
     if (threadIdx.x < kWave) {
 #pragma unroll
@@ -936,7 +1183,7 @@ __global__ __launch_bounds__(BS) void k_reduce_col2d(const T* __restrict__ a, Co
     }
     A acc[VEC];
     T first[VEC];
-    col_partial<Op, T, VEC, UNROLL, BS>(a, ca, vec_ok, t, cg, 0, part, acc, first);
+    col_partial<Op, T, VEC, UNROLL, BS>(a, ca, t, cg, 0, part, acc, first);
     if (threadIdx.x < kWave) {  // wave 0 holds the block's per-column results
       AF best = OpF::init();
 #pragma unroll
@@ -1357,11 +1604,95 @@ inline RowIndexer<1> out_indexer(const ReducePlan& p, int ndims) {
   return ix;
 }
 
+// How a column reduction (strided axis, unit-stride outputs) runs:
+//  * lanes, when one lane per 16 bytes of outputs makes at least 32768 lanes (two waves per CU):
+//    (512, 16, 2048) f32 over axis 1: max 24.5 -> 13.7 us, sum 14.7 -> 13.6;
+//  * spans, for rows of up to 4 KB (sums) or less than 4 KB (max / min / arg) that a block of at most
+//    512 lanes can cover with a whole number of rows per step.  256 blocks (one per CU, 8 x 16-byte
+//    loads in flight per lane, twice buffered) ran faster than 512 and 1024: (1000003, 37) f32 mean
+//    444 (column kernel) -> 30.8 us, against 32.8 and 36.2; max 941 -> 33.8; (131072, 384) f32 mean
+//    55.9 -> 36, against 45.7 with 512.  Rows of exactly 4 KB: (32768, 1024) f32 mean 38.3 -> 28.8 us,
+//    but max 29.8 -> 31.4.  Inputs of at most 4 MB split by column strips instead of row tiles, which
+//    saves the second launch ((300, 700) f32 sum 6.7 -> 4.4 us, 6.8 with row tiles; at 25 MB the
+//    strips' short runs cost more than the launch: (64, 1000, 100) 14.1 against 10.4 us);
+//  * the 64-lane column kernel otherwise.
+struct ColRoute {
+  enum : int { kColumns = 0, kLanes = 1, kSpans = 2 };
+  int kind = kColumns;
+  uint32_t bs = 0, cw = 0, strips = 1, m = 0, lanes = 0, tiles = 1;
+  bool flat = false;
+};
+constexpr uint64_t kLaneItems = 32768;
+constexpr uint64_t kSpanRowBytes = 4096;
+constexpr uint64_t kSpanBlocks = 256;
+constexpr uint64_t kSpanStripBytes = uint64_t(4) << 20;
+
+inline uint32_t gcd32(uint32_t a, uint32_t b) { return b == 0 ? a : gcd32(b, a % b); }
+
+inline ColRoute col_route(const ReducePlan& p, size_t es, bool ordered) {
+  ColRoute r;
+  const uint32_t V = es >= 16 ? 1 : uint32_t(16 / es);
+  const uint64_t C = p.oshape[p.ond - 1];
+  const uint64_t outer = p.out_size / C;
+  if (p.kind != kColReduce || p.R >= (uint64_t(1) << 31) || C >= (uint64_t(1) << 31)) return r;
+  // the outer dims are decoded in 32 bits
+  if (outer >= (uint64_t(1) << 31)) return r;
+  const uint64_t items = outer * ceil_div(C, V);
+  if (C >= V && items >= kLaneItems && items < (uint64_t(1) << 31)) {
+    r.kind = ColRoute::kLanes;
+    return r;
+  }
+  if (C * es > kSpanRowBytes || (ordered && C * es == kSpanRowBytes)) return r;
+  const bool contiguous = p.rstride == int64_t(C);
+  if ((C % V != 0 && !contiguous) || p.R * C < V) return r;
+  const uint64_t round = uint64_t(kSpanBS) * kSpanUnroll * V;  // elements of one round of a whole block
+  uint64_t cw = C;
+  if (C % V == 0 && outer < kSpanBlocks && p.R * C > round && outer * p.R * C * es <= kSpanStripBytes) {
+    cw = C / ceil_div(kSpanBlocks, outer) / V * V;
+    const uint64_t least = 64 / es;  // 64-byte runs
+    if (cw < least) cw = least;
+    if (cw > C) cw = C;
+  }
+  const uint32_t period = uint32_t(cw) / gcd32(uint32_t(cw), V);  // lanes of the shortest whole-row step
+  if (period > uint32_t(kSpanBS)) return r;
+  r.cw = uint32_t(cw);
+  r.strips = uint32_t(ceil_div(C, cw));
+  if (outer * r.strips * kSpanBlocks >= (uint64_t(1) << 31)) return r;
+  r.kind = ColRoute::kSpans;
+  r.flat = contiguous && r.strips == 1;
+  // the block size with the fewest idle lanes, no larger than one round of the slice needs
+  uint64_t most = ceil_div(ceil_div(p.R * cw, uint64_t(V) * kSpanUnroll), kWave) * kWave;
+  const uint64_t least = ceil_div(period, kWave) * kWave;
+  if (most < least) most = least;
+  if (most > uint64_t(kSpanBS)) most = kSpanBS;
+  for (uint32_t bs = uint32_t(most); bs >= least && 2 * bs > most; bs -= kWave) {
+    const uint32_t n = bs / period * period;
+    if (r.bs == 0 || uint64_t(n) * r.bs > uint64_t(r.lanes) * bs + uint64_t(r.bs) * bs / 50) {
+      r.bs = bs;
+      r.lanes = n;
+    }
+  }
+  r.m = uint32_t(uint64_t(r.lanes) * V / cw);
+  // a second launch folds the tiles: not worth it below 6 rounds
+  const uint64_t chunks = p.R / (uint64_t(r.m) * kSpanUnroll);
+  uint64_t tiles = ceil_div(kSpanBlocks, outer * r.strips);
+  if (tiles > chunks / 2) tiles = chunks / 2;
+  // the partials (at most 2 * es bytes each) have to fit the 1 MiB workspace of a stream
+  const uint64_t room = (uint64_t(1) << 20) / (p.out_size * 2 * es);
+  if (tiles > room) tiles = room;
+  r.tiles = uint32_t(chunks < 6 || tiles < 1 ? 1 : tiles);
+  return r;
+}
+
 // Recommended tiles per output: enough (output, tile) work items to fill 256 CUs several times
 // over while each tile still streams a few tens of KB.
 inline size_t tiles_hint(const ReducePlan& p, size_t es) {
   if (p.R <= 1 || p.out_size == 0) return 1;
   if (p.kind == kColReduce) {
+    // (rows of exactly 4 KB, where sums and ordered ops part, take the column kernel's tiles here)
+    const ColRoute route = col_route(p, es, true);
+    if (route.kind == ColRoute::kLanes) return 1;
+    if (route.kind == ColRoute::kSpans) return route.tiles;
     // column tiles: ~256 long-lived blocks (one per CU, 8 loads of 16 bytes in flight per lane)
     // measured best: (8192, 8192) f32 axis 0 at 6.3 TB/s vs 6.0 with 512 blocks of 4 loads;
     // more concurrent row bands lose to HBM row conflicts (32 bands: 4.7-5.6 TB/s); >= 64 rows
@@ -1388,6 +1719,38 @@ inline size_t tiles_hint(const ReducePlan& p, size_t es) {
   return size_t(tiles < 1 ? 1 : tiles);
 }
 
+// The span route in one launch (one tile) or two (partials in `part`, folded and zeroed by the
+// second); `part_bytes` limits the tiles.
+template <class Op, class T>
+void launch_reduce_span(const T* a, RedOut<T> out, const ReducePlan& p, const ColRoute& r, typename Op::A* part,
+                        size_t part_bytes, hipStream_t st) {
+  constexpr int V = rvec<T>();
+  SpanArgs sa{};
+  sa.ix = out_indexer(p, p.ond - 1);
+  sa.C = uint32_t(p.oshape[p.ond - 1]);
+  sa.cw = r.cw;
+  sa.strips = r.strips;
+  sa.m = r.m;
+  sa.lanes = r.lanes;
+  const uint64_t room = part_bytes / (p.out_size * sizeof(typename Op::A));
+  sa.tiles = room < r.tiles ? uint32_t(room < 1 ? 1 : room) : r.tiles;
+  sa.R = p.R;
+  sa.rs = p.rstride;
+  sa.whole = uint32_t(p.R / (uint64_t(r.m) * kSpanUnroll));
+  sa.flat = r.flat;
+  const uint64_t outer = p.out_size / sa.C;
+  const dim3 grid(unsigned(outer * sa.strips * sa.tiles));
+  if (sa.tiles == 1) {
+    k_reduce_span<Op, T, V, kSpanUnroll, true><<<grid, r.bs, 0, st>>>(a, sa, out, part);
+    return;
+  }
+  k_reduce_span<Op, T, V, kSpanUnroll, false><<<grid, r.bs, 0, st>>>(a, sa, out, part);
+  const uint32_t cb = sa.C < 32 ? sa.C : 32;
+  const uint32_t groups = uint32_t(ceil_div(sa.C, cb));
+  k_span_final<Op, T><<<dim3(unsigned(outer * groups)), kSpanBS, 0, st>>>(a, part, sa.ix, sa.C, sa.tiles, cb, groups,
+                                                                         out);
+}
+
 template <class Op, class T, int WRITE>
 void launch_reduce(const T* a, RedOut<T> out, int ndim, const size_t* shape, const ssize_t* strides, int axis,
                    size_t axis_len, size_t out_size, size_t tiles, hipStream_t st) {
@@ -1406,6 +1769,23 @@ void launch_reduce(const T* a, RedOut<T> out, int ndim, const size_t* shape, con
   // reductions write next to nothing, so streaming loads win at every volume measured (the
   // 128 MB c64 sum: 5.1 TB/s streaming vs 4.6 default), unlike the elementwise kernels
   const bool nt = true;
+  if constexpr (WRITE == kWriteFinal) {
+    if (tiles == 1 && p.R > 0) {
+      const ColRoute r = col_route(p, sizeof(T), Op::kOrdered);
+      if (r.kind == ColRoute::kLanes) {
+        const uint32_t C = uint32_t(p.oshape[p.ond - 1]);
+        const uint32_t vpr = uint32_t(ceil_div(C, V));
+        const uint32_t items = uint32_t(p.out_size / C * vpr);
+        k_reduce_lane<Op, T, V, kSpanUnroll><<<dim3(unsigned(ceil_div(items, kRBlock))), kRBlock, 0, st>>>(
+            a, out_indexer(p, p.ond - 1), C, make_fastdiv(vpr), p.R, p.rstride, items, out);
+        return;
+      }
+      if (r.kind == ColRoute::kSpans) {
+        launch_reduce_span<Op, T>(a, out, p, r, nullptr, 0, st);
+        return;
+      }
+    }
+  }
   if (p.kind == kColReduce && p.oshape[p.ond - 1] < (uint64_t(1) << 31)) {
     ColArgs ca{};
     ca.nt = nt;
@@ -1416,17 +1796,14 @@ void launch_reduce(const T* a, RedOut<T> out, int ndim, const size_t* shape, con
     ca.rs = p.rstride;
     ca.chunk = ceil_div(p.R, tiles);
     ca.tiles = uint32_t(tiles);
-    bool vec_ok = al16(a) && (ca.C % V == 0) && ((uint64_t(p.rstride < 0 ? -p.rstride : p.rstride) * sizeof(T)) % 16 == 0);
-    for (int d = 0; d < p.ond - 1; ++d)
-      if ((uint64_t(p.ostride[d] < 0 ? -p.ostride[d] : p.ostride[d]) * sizeof(T)) % 16) vec_ok = false;
     const uint64_t blocks = (p.out_size / ca.C) * ca.cgroups * ca.tiles;
     // sums: 8 waves with 4 rows of loads each (42.4-42.7 us for the (8192, 8192) f32 axis-0
     // partial, against 43.4-43.9 with 4 waves x 8 rows); ordered ops keep 4 waves x 8 rows
     // (46.0 us, against 46.9-47.3 with 8 waves): their pipelined fold wants the registers
     if constexpr (Op::kOrdered)
-      k_reduce_col<Op, T, V, 8, WRITE, 256><<<dim3(unsigned(blocks)), 256, 0, st>>>(a, ca, out, vec_ok);
+      k_reduce_col<Op, T, V, 8, WRITE, 256><<<dim3(unsigned(blocks)), 256, 0, st>>>(a, ca, out);
     else
-      k_reduce_col<Op, T, V, 4, WRITE, 512><<<dim3(unsigned(blocks)), 512, 0, st>>>(a, ca, out, vec_ok);
+      k_reduce_col<Op, T, V, 4, WRITE, 512><<<dim3(unsigned(blocks)), 512, 0, st>>>(a, ca, out);
     return;
   }
   RowArgs ra{};
@@ -1523,9 +1900,6 @@ int launch_reduce_col_last(const T* a, RedOut<T> out, const ReducePlan& p, size_
   ca.rs = p.rstride;
   ca.chunk = ceil_div(p.R, uint64_t(tiles));
   ca.tiles = uint32_t(tiles);
-  bool vec_ok = al16(a) && (ca.C % V == 0) && ((uint64_t(p.rstride < 0 ? -p.rstride : p.rstride) * sizeof(T)) % 16 == 0);
-  for (int d = 0; d < p.ond - 1; ++d)
-    if ((uint64_t(p.ostride[d] < 0 ? -p.ostride[d] : p.ostride[d]) * sizeof(T)) % 16) vec_ok = false;
   const uint64_t groups = (p.out_size / ca.C) * ca.cgroups;
   const uint64_t blocks = groups * tiles;
   const uint64_t slot_words = groups * tiles * uint64_t(kWave) * V * W;
@@ -1536,7 +1910,7 @@ int launch_reduce_col_last(const T* a, RedOut<T> out, const ReducePlan& p, size_
   fa.fault = w.fault;
   fa.spin_limit = wait_spin_limit();
   uint32_t* counters = reinterpret_cast<uint32_t*>(fa.slots + slot_words);
-  k_reduce_col_last<Op, T, V, 4, 512><<<dim3(unsigned(blocks)), 512, 0, st>>>(a, ca, out, vec_ok, fa, counters);
+  k_reduce_col_last<Op, T, V, 4, 512><<<dim3(unsigned(blocks)), 512, 0, st>>>(a, ca, out, fa, counters);
   return kFusedLaunched;
 }
 
@@ -1551,6 +1925,17 @@ int launch_reduce_fused(const T* a, RedOut<T> out, int ndim, const size_t* shape
   if (!args_ok(ndim, axis)) return kFusedNotCovered;
   ReducePlan p;
   plan_reduce(p, ndim, shape, strides, axis, axis_len, out_size);
+  if (p.kind == kColReduce) {
+    const ColRoute r = col_route(p, sizeof(T), Op::kOrdered);
+    if (r.kind == ColRoute::kLanes) {
+      launch_reduce<Op, T, kWriteFinal>(a, out, ndim, shape, strides, axis, axis_len, out_size, 1, st);
+      return kFusedLaunched;
+    }
+    if (r.kind == ColRoute::kSpans) {
+      launch_reduce_span<Op, T>(a, out, p, r, reinterpret_cast<typename Op::A*>(w.payload), w.payload_bytes, st);
+      return kFusedLaunched;
+    }
+  }
   if constexpr (!Op::kOrdered) {
     if (p.kind == kColReduce) return launch_reduce_col_last<Op, T>(a, out, p, tiles, w, st);
   }
@@ -1719,7 +2104,6 @@ int launch_reduce_2d_ordered(const T* a, RedOut<T> out, uint64_t R, uint64_t C, 
   ca.chunk = ceil_div(R, tiles);
   ca.tiles = uint32_t(tiles);
   const uint32_t nblk = uint32_t(uint64_t(ca.cgroups) * tiles);
-  const bool vec_ok = al16(a) && (C % V == 0) && (C * sizeof(T)) % 16 == 0;
   const uint64_t W = sizeof(typename OpF::A) / 4;
   if (uint64_t(nblk) * W * 8 > w.payload_bytes) return kFusedNoRoom;
   FusedArgs fa{};
@@ -1728,9 +2112,9 @@ int launch_reduce_2d_ordered(const T* a, RedOut<T> out, uint64_t R, uint64_t C, 
   fa.spin_limit = wait_spin_limit();
   const dim3 g(nblk + 1);
   switch (ceil_div(nblk, uint64_t(BS))) {
-    case 1: k_reduce_col2d<Op, OpF, T, V, 8, BS, 1><<<g, BS, 0, st>>>(a, ca, nblk, vec_ok, out, fa); break;
-    case 2: k_reduce_col2d<Op, OpF, T, V, 8, BS, 2><<<g, BS, 0, st>>>(a, ca, nblk, vec_ok, out, fa); break;
-    default: k_reduce_col2d<Op, OpF, T, V, 8, BS, 4><<<g, BS, 0, st>>>(a, ca, nblk, vec_ok, out, fa); break;
+    case 1: k_reduce_col2d<Op, OpF, T, V, 8, BS, 1><<<g, BS, 0, st>>>(a, ca, nblk, out, fa); break;
+    case 2: k_reduce_col2d<Op, OpF, T, V, 8, BS, 2><<<g, BS, 0, st>>>(a, ca, nblk, out, fa); break;
+    default: k_reduce_col2d<Op, OpF, T, V, 8, BS, 4><<<g, BS, 0, st>>>(a, ca, nblk, out, fa); break;
   }
   return kFusedLaunched;
 }

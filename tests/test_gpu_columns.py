@@ -1,0 +1,95 @@
+"""GPU parity of column reductions (a strided axis with unit-stride outputs) at the edges of their
+kernels: whole-row steps over narrow rows (the period of odd row lengths, masked last rounds, column
+strips, several tiles folded by a second launch), one lane per output vector, and rows of odd length
+in the 64-lane column kernel.  Bounds as in test_gpu_reduce.py."""
+import numpy as np
+import pytest
+
+import musapy_amd as ms
+from oracle import reference as R
+from tests.conftest import assert_bits_equal
+from tests.test_gpu_reduce import check_reduce, dev
+
+pytestmark = pytest.mark.gpu
+RNG = np.random.default_rng(4711)
+
+# (shape, axis): what the shape reaches
+SHAPES = [
+    ((7, 2), 0), ((2, 3), 0), ((1, 5), 0),                      # a slice of less than one step
+    ((50000, 2), 0), ((20000, 3), 0), ((9001, 37), 0),          # short periods, several tiles
+    ((1500, 511), 0), ((1501, 257), 0),                         # periods near a whole block
+    ((4097, 96), 0), ((300, 700), 0), ((257, 640), 0),          # column strips, the last one narrower
+    ((900, 1024), 0), ((900, 1020), 0), ((301, 1025), 0),       # either side of 4 KB rows (f32)
+    ((130, 4099), 0), ((3, 100, 130), 1),                       # odd rows of the column kernel
+    ((9, 500, 5), 1), ((40, 33, 7), 1), ((300, 6, 13), 1),      # many short slices
+    ((70, 5, 2001), 1), ((2, 3, 70001), 1),                     # one lane per output vector
+]
+
+
+def values(kind, dt, shape):
+    if dt == np.int64:
+        return RNG.integers(-1000, 1000, shape).astype(np.int64)
+    x = RNG.uniform(0.999, 1.001, shape) if kind == "prod" else RNG.standard_normal(shape)
+    if dt in (np.complex64, np.complex128):
+        x = x + 1j * RNG.standard_normal(shape) * (1e-3 if kind == "prod" else 1)
+    return x.astype(dt)
+
+
+KINDS = [(k, d) for d in (np.float32, np.float64, np.int64) for k in ("sum", "mean", "max", "argmin")]
+KINDS += [("prod", np.float32), ("min", np.float32), ("argmax", np.float64)]
+KINDS += [(k, d) for d in (np.complex64, np.complex128) for k in ("sum", "mean")]
+
+
+@pytest.mark.parametrize("kind,dt", KINDS, ids=[f"{k}-{np.dtype(d).name}" for k, d in KINDS])
+def test_column_shapes(kind, dt):
+    for shape, axis in SHAPES:
+        check_reduce(kind, values(kind, dt, shape), axis)
+
+
+@pytest.mark.parametrize("kind", ["max", "min", "argmax", "argmin"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_column_ordered_semantics(kind, dt):
+    """Ties, both zeros, a NaN in row 0 (absorbs the column), later NaNs, all-NaN columns, infinities."""
+    for shape, axis in SHAPES:
+        x = RNG.integers(-2, 3, shape).astype(dt)
+        y = np.moveaxis(x, axis, 0)
+        n = y.shape[0]
+        y[n // 2][..., 1::3] = np.nan
+        y[0][..., ::5] = np.nan
+        y[-1][..., 2::7] = -0.0
+        if n > 2:
+            y[1:, ..., -1] = np.nan
+            y[0][..., -1] = -np.inf
+        check_reduce(kind, x, axis)
+    z = np.full((9001, 37), np.nan, dt)
+    z[0] = np.inf if kind.endswith("min") else -np.inf
+    check_reduce(kind, z, 0)
+
+
+@pytest.mark.parametrize("kind", ["sum", "max", "argmin"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_column_views(kind, dt):
+    """Rows that are not contiguous, reversed rows of the axis, and bases off 16-byte alignment."""
+    base = RNG.standard_normal((3001, 133)).astype(dt)
+    B = dev(base)
+    for lo, hi in ((0, 64), (1, 65), (3, 103), (5, 42), (2, 133)):
+        check_reduce(kind, np.ascontiguousarray(base[:, lo:hi]), 0, gpu_x=ms.slice(B, [(0, 3001, 1), (lo, hi, 1)]))
+        check_reduce(kind, np.ascontiguousarray(base[1::2, lo:hi]), 0, gpu_x=ms.slice(B, [(1, 3001, 2), (lo, hi, 1)]))
+    check_reduce(kind, np.ascontiguousarray(base[::-1]), 0, gpu_x=ms.flip(B, 0))
+    flat = RNG.standard_normal(3001 * 37 + 1).astype(dt)
+    F = dev(flat)
+    view = ms.slice(F, [(1, flat.size, 1)])  # 4 or 8 bytes past 16-byte alignment
+    check_reduce(kind, flat[1:], None, gpu_x=view)
+
+
+def test_column_results_repeat():
+    """The same bits on every call, and with other reductions on the workspace in between."""
+    x = RNG.standard_normal((40001, 37)).astype(np.float32)
+    X = dev(x)
+    first = [ms.sum(X, axis=0).numpy(), ms.argmax(X, axis=0).numpy()]
+    for _ in range(3):
+        ms.sum(X)
+        assert_bits_equal(ms.sum(X, axis=0).numpy(), first[0], "sum")
+        ms.max(X, axis=(0, 1))
+        assert_bits_equal(ms.argmax(X, axis=0).numpy(), first[1], "argmax")
+    assert_bits_equal(first[1], R.reduce(x, "argmax", 0), "argmax against the oracle")
