@@ -360,9 +360,13 @@ int musapy_reduce_fused_v1(int op, int dtype, const void* a, void* c, int ndim, 
  * musapy_cumsum_ws_v2: every cumsum, with its waits reported to the fault word of `workspace`:
  * the chained scan on the workspace's payload when it fits (else on `tmp`, cleared first), the
  * look-back of fewer rows on `tmp` (its claim counter and status words, cleared by the launch),
- * the sequential scan of a strided axis with neither.  `tmp` may be NULL when the shape takes
- * no scratch; a `tmp` of the _v3 formula's capacity always suffices.  Returns 0 when launched, -1
- * when not (wrapper error 1: tmp missing or too small for the path taken; 3 or 4 as for _v3). */
+ * the look-back of a strided axis on `tmp` too (without one, or with one that is too small, that
+ * axis runs one lane per column vector), other strided axes with neither.  `tmp` may be NULL when
+ * the shape takes no scratch; a `tmp` of the _v3 formula's capacity always suffices.  Returns 0 when launched, -1
+ * when not (wrapper error 1: tmp missing or too small for the path taken; 3 or 4 as for _v3).
+ * musapy_cumsum_scratch_v1: the bytes of `tmp` with which musapy_cumsum_ws_v2 takes its fastest
+ * path for a call, given a workspace of `workspace_bytes` (0: none needed). */
+size_t musapy_cumsum_scratch_v1(int dtype, int ndim, const size_t* in_shape, const ssize_t* in_strides, int axis, size_t axis_len, size_t out_size, size_t workspace_bytes);
 int musapy_cumsum_ws_v1(int dtype, const void* a, void* c, int ndim, const size_t* in_shape, const ssize_t* in_strides, int axis, size_t axis_len, size_t out_size, void* workspace, size_t workspace_bytes, hipStream_t stream);
 int musapy_cumsum_ws_v2(int dtype, const void* a, void* c, void* tmp, size_t tmp_bytes, int ndim, const size_t* in_shape, const ssize_t* in_strides, int axis, size_t axis_len, size_t out_size, void* workspace, size_t workspace_bytes, hipStream_t stream);
 

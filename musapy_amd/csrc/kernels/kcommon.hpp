@@ -150,6 +150,23 @@ __device__ inline void vstore_nt(T* p, const Vec<T, N>& v) {
 // Reductions always stream (they write next to nothing).
 constexpr uint64_t kStreamLoadBytes = uint64_t(32) << 20;
 
+// The store counterpart of vload_el.
+template <bool NT, typename T, int N>
+__device__ inline void vstore_el(T* p, const Vec<T, N>& v) {
+  constexpr int kB = int(sizeof(T) * N);
+  constexpr int kW = kB > 16 ? 16 : kB;
+  constexpr int kA = int(alignof(T)) < kW ? int(alignof(T)) : kW;
+  using W = typename NtWord<kW>::type;
+  using U = typename ElWord<kW, kA>::type;
+  W w[kB / kW];
+  __builtin_memcpy(w, &v, kB);
+#pragma unroll
+  for (int i = 0; i < kB / kW; ++i) {
+    if constexpr (NT) __builtin_nontemporal_store(w[i], reinterpret_cast<U*>(p) + i);
+    else reinterpret_cast<U*>(p)[i] = w[i];
+  }
+}
+
 template <typename T, int N>
 __device__ inline Vec<T, N> vload_pol(const T* p, bool nt) {
   return nt ? vload_nt<T, N>(p) : vload<T, N>(p);

@@ -13,11 +13,12 @@
 //              188 us with 16 KB tiles and 237 us for one block per row walking it tile by tile (the
 //              previous design, whose one-block-per-row access pattern topped out at the rate of a
 //              plain copy in that pattern).
-//   col        the axis is strided but the innermost other dim is unit-stride: lanes walk
-//              adjacent columns, each carrying a running sum down the axis (coalesced,
-//              sequential order).
-//   generic    one lane per row, sequential along the axis (any strides).
-// col and generic add in exactly the reference CPU order (acc = 0; acc += x[k]).  The tiled
+//   cols       the axis is strided but the innermost other dim is unit-stride: tiles of 256-byte
+//              runs of columns, with a decoupled look-back down the columns.  (8192, 4096) f32 over
+//              axis 0: 54 us, against 925 us with one lane per column.
+//   lane       the same layout with a short axis or very many columns: one lane per column.
+//   sequential one lane per row along the axis (any strides, and the shortest or widest columns).
+// lane and sequential add in exactly the reference CPU order (acc = 0; acc += x[k]).  The tiled
 // paths fix their association by the tile shape, so results are the same bits run to run.
 #include "kcommon.hpp"
 #include "publish.hpp"
@@ -80,6 +81,10 @@ __device__ inline A wave_incl_scan_dpp(A v) {
   v = v + dpp_move<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
   return v;
 }
+// the value of the lane `s` lanes below
+__device__ inline float shfl_up(float v, int s) { return __shfl_up(v, s, kWave); }
+__device__ inline double shfl_up(double v, int s) { return __shfl_up(v, s, kWave); }
+__device__ inline uint64_t shfl_up(uint64_t v, int s) { return __shfl_up((unsigned long long)v, s, kWave); }
 template <class A>
 __device__ inline A wave_shr1(A v) { return dpp_move<0x138>(v); }  // wave_shr:1, lane 0 gets 0
 // the value of lane `l` (uniform), through scalar registers
@@ -449,6 +454,239 @@ __global__ __launch_bounds__(BS) void k_scan_chain(const T* __restrict__ a, T* _
 }
 
 // ---------------------------------------------------------------------------------------------
+// Column scan with a decoupled look-back, for a strided axis whose other innermost dim is
+// unit-stride.  A tile is LPC * VE columns (LPC lanes of one 16-byte vector each: 256-byte runs)
+// by (BS / LPC) * RPL rows; lane (group g, column vector) holds RPL consecutive rows, scans them in
+// registers, and the groups' totals meet through wave shifts and LDS.  Wave 0 then handles one
+// column per lane: it publishes the tile's aggregate, looks back over up to kColWindow
+// predecessors at once for the nearest published prefix, P(t - 1) = ((P(j) + A(j + 1)) + ...) +
+// A(t - 1), and publishes P(t).  Each status word holds 32 bits of a value, the published tag and a
+// flag that tells a prefix from an aggregate; the prefix replaces the aggregate in place, so a
+// predecessor costs one read.  The fold follows P(t) = P(t - 1) + A(t) whichever j is found: the
+// same bits run to run.  Blocks are numbered tile-major over the strips, whose count is rounded up
+// to a multiple of 8, so a tile's predecessors sit earlier on the same XCD (see k_scan_chain) and
+// are resident or finished; within a tile row each XCD takes neighbouring strips, which share the
+// lines at their edges in its L2 ((8192, 4097) f32 88 -> 67 us with default stores, (16384, 16384)
+// 403 -> 364 us).  Waits are bounded as in the other scans.
+// It is bound by its memory traffic: 51.8 us of kernel time for (8192, 4096) f32 (5.2 TB/s), 93.2 for
+// f64 (5.8 TB/s); a window of 16 predecessors costs registers and ran 62.7 us.
+struct ColScanArgs {
+  RowIndexer<2> ix;     // outer dims: [0] input, [1] output strides
+  uint64_t L;
+  uint64_t C;           // innermost extent (unit stride on both sides)
+  int64_t ls_in, ls_out;
+  FastDiv gdiv;         // divides a tile id by the groups per tile row (a multiple of 8 without claims)
+  FastDiv sdiv;         // divides a group by the strips per outer slice
+  uint32_t groups;      // strips of all outer slices
+  uint32_t* counter;    // tile claims, when the groups are few; else nullptr
+  uint32_t tiles;       // tiles down the axis
+  uint64_t* status;     // per (group, tile, column): W words
+  uint32_t* fault;
+  uint32_t spin_limit;
+  bool nt_load;
+};
+constexpr int kColWindow = 8;
+constexpr uint64_t kPrefixFlag = uint64_t(1) << 33;
+
+template <class T, int VE, int BS, int RPL, int LPC, bool CLAIM, bool NTS>
+__global__ __launch_bounds__(BS) void k_scan_cols(const T* __restrict__ a, T* __restrict__ c, ColScanArgs sa) {
+  using A = typename ScanAcc<T>::A;
+  constexpr int SC = LPC * VE;              // columns of a tile
+  constexpr int kWaves = BS / kWave;
+  constexpr int TR = BS / LPC * RPL;        // rows of a tile
+  constexpr int W = sizeof(A) == 4 ? 1 : 2;
+  static_assert(SC <= kWave, "one lane of wave 0 per column");
+  __shared__ A s_w[kWaves][SC];
+  const int tid = threadIdx.x, lane = tid % kWave, wv = tid / kWave;
+  uint32_t id = blockIdx.x;
+  if constexpr (CLAIM) {
+    __shared__ uint32_t s_id;
+    if (tid == 0) s_id = atomicAdd(sa.counter, 1u);
+    __syncthreads();
+    id = s_id;
+  }
+  const uint32_t t = fd_div(sa.gdiv, id);
+  const uint32_t gb = id - t * sa.gdiv.d;
+  const uint32_t g = CLAIM ? gb : (gb % 8) * (sa.gdiv.d / 8) + gb / 8;
+  if (g >= sa.groups) return;
+  const uint32_t outer = fd_div(sa.sdiv, g);
+  const uint32_t strip = g - outer * sa.sdiv.d;
+  int64_t off[2];
+  row_offsets<2>(sa.ix, outer, off);
+  const int lc = tid % LPC;
+  // the last vector of an odd row moves back to end with it; lanes past the row read column 0 on
+  uint64_t c0 = uint64_t(strip) * SC + uint64_t(lc) * VE;
+  const bool live = c0 < sa.C;
+  if (!live) c0 = 0;
+  if (c0 + VE > sa.C) c0 = sa.C - VE;
+  const uint64_t r0 = uint64_t(t) * TR + uint64_t(tid / LPC) * RPL;
+  const T* ip = a + off[0] + int64_t(c0);
+  Vec<T, VE> d[RPL];
+#pragma unroll
+  for (int i = 0; i < RPL; ++i) {
+    const uint64_t r = r0 + i < sa.L ? r0 + i : sa.L - 1;
+    d[i] = vload_el<T, VE>(ip + int64_t(r) * sa.ls_in, sa.nt_load);
+  }
+  A x[RPL][VE];
+#pragma unroll
+  for (int i = 0; i < RPL; ++i)
+#pragma unroll
+    for (int e = 0; e < VE; ++e) {
+      const A v = r0 + i < sa.L ? A(d[i].v[e]) : A(0);
+      x[i][e] = i == 0 ? A(0) + v : x[i - 1][e] + v;
+    }
+  A ex[VE];  // sum of the earlier groups of the wave
+#pragma unroll
+  for (int e = 0; e < VE; ++e) {
+    A incl = x[RPL - 1][e];
+#pragma unroll
+    for (int s = LPC; s < kWave; s *= 2) {
+      const A y = shfl_up(incl, s);
+      if (lane >= s) incl = y + incl;
+    }
+    if (lane >= kWave - LPC) s_w[wv][lc * VE + e] = incl;
+    const A y = shfl_up(incl, LPC);
+    ex[e] = lane >= LPC ? y : A(0);
+  }
+  lds_barrier();
+  if (tid < SC) {  // one column per lane of wave 0
+    A w[kWaves];
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) w[i] = s_w[i][tid];
+    A agg = w[0];
+#pragma unroll
+    for (int i = 1; i < kWaves; ++i) agg = agg + w[i];
+    A P = A(0);
+    if (sa.tiles > 1) {
+      uint64_t* const st = sa.status + (uint64_t(g) * sa.tiles * SC + tid) * W;  // tile 0's words of this column
+      constexpr uint64_t kNext = uint64_t(SC) * W;
+      const bool last = t + 1 == sa.tiles;  // nothing waits on the last tile
+      auto publish = [&](A v, uint64_t flag) {
+        const uint64_t b = bits_of(v);
+        st_relaxed(st + t * kNext, kTag | flag | (b & 0xffffffffu));
+        if (W == 2) st_relaxed(st + t * kNext + 1, kTag | flag | (b >> 32));
+      };
+      if (t > 0) {
+        if (!last) publish(agg, 0);
+        bool found = false;
+        for (uint32_t spins = 0; !found && spins < sa.spin_limit; ++spins) {
+          uint64_t q[kColWindow][W];
+#pragma unroll
+          for (int j = 0; j < kColWindow; ++j)
+#pragma unroll
+            for (int k = 0; k < W; ++k) q[j][k] = uint32_t(j) < t ? ld_relaxed(st + (t - 1 - j) * kNext + k) : 0;
+          bool open = true;  // every nearer tile has published its aggregate
+          int li = -1;       // the nearest tile with a prefix
+#pragma unroll
+          for (int j = 0; j < kColWindow; ++j) {
+            bool tag = true, inc = true, agr = true;
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+              tag = tag && (q[j][k] & kTag);
+              inc = inc && (q[j][k] & kPrefixFlag);
+              agr = agr && !(q[j][k] & kPrefixFlag);
+            }
+            if (open && li < 0 && tag && inc) li = j;
+            open = open && tag && agr;  // halves of an aggregate and of a prefix: read again
+          }
+          if (li >= 0) {
+            found = true;
+#pragma unroll
+            for (int j = kColWindow - 1; j >= 0; --j) {
+              uint64_t b = 0;
+#pragma unroll
+              for (int k = 0; k < W; ++k) b |= (q[j][k] & 0xffffffffu) << (32 * k);
+              if (j == li) P = from_bits<A>(b);
+              else if (j < li) P = P + from_bits<A>(b);
+            }
+          } else {
+            __builtin_amdgcn_s_sleep(1);
+          }
+        }
+        if (!found) atomicOr(sa.fault, kFaultScanWait);  // the prefix stays 0
+      }
+      if (!last) publish(P + agg, kPrefixFlag);
+    }
+    A run = P;  // the column's sum before each wave's rows
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) {
+      s_w[i][tid] = run;
+      run = run + w[i];
+    }
+  }
+  lds_barrier();
+  if (!live) return;
+  T* op = c + off[1] + int64_t(c0);
+#pragma unroll
+  for (int e = 0; e < VE; ++e) ex[e] = s_w[wv][lc * VE + e] + ex[e];
+#pragma unroll
+  for (int i = 0; i < RPL; ++i) {
+    if (r0 + i >= sa.L) break;
+    Vec<T, VE> v;
+#pragma unroll
+    for (int e = 0; e < VE; ++e) v.v[e] = T(ex[e] + x[i][e]);
+    vstore_el<NTS, T, VE>(op + int64_t(r0 + i) * sa.ls_out, v);
+  }
+}
+
+// One lane per column, sequential along the axis in the reference's order (acc = 0; acc += x[k]):
+// short axes, and scans with enough columns to fill the GPU.  The next U rows are in flight while U
+// rows are added and stored.
+template <class T, int U, bool NTS>
+__global__ __launch_bounds__(kSBlock) void k_scan_lane(const T* __restrict__ a, T* __restrict__ c, ColScanArgs sa,
+                                                       FastDiv cdiv, uint32_t cols) {
+  using A = typename ScanAcc<T>::A;
+  const uint32_t it = blockIdx.x * kSBlock + threadIdx.x;
+  if (it >= cols) return;
+  const uint32_t outer = fd_div(cdiv, it);
+  const uint32_t c0 = it - outer * cdiv.d;
+  int64_t off[2];
+  row_offsets<2>(sa.ix, outer, off);
+  const T* ip = a + off[0] + c0;
+  T* op = c + off[1] + c0;
+  A acc = A(0);
+  Vec<T, 1> x[U], y[U];
+  // whole rounds without conditions; only the last one is masked (its loads read the last row)
+  auto load = [&](uint64_t k, Vec<T, 1>(&d)[U]) {
+    if (k + U <= sa.L) {
+      const T* q = ip + int64_t(k) * sa.ls_in;
+#pragma unroll
+      for (int u = 0; u < U; ++u) d[u] = vload_pol<T, 1>(q + int64_t(u) * sa.ls_in, sa.nt_load);
+    } else if (k < sa.L) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint64_t r = k + u < sa.L ? k + u : sa.L - 1;
+        d[u] = vload_pol<T, 1>(ip + int64_t(r) * sa.ls_in, sa.nt_load);
+      }
+    }
+  };
+  auto add_row = [&](const Vec<T, 1>& d, T* q) {
+    acc = acc + A(d.v[0]);
+    Vec<T, 1> v;
+    v.v[0] = T(acc);
+    vstore_as<NTS, T, 1>(q, v);
+  };
+  auto add = [&](uint64_t k, const Vec<T, 1>(&d)[U]) {
+    T* q = op + int64_t(k) * sa.ls_out;
+    if (k + U <= sa.L) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) add_row(d[u], q + int64_t(u) * sa.ls_out);
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (k + u < sa.L) add_row(d[u], q + int64_t(u) * sa.ls_out);
+    }
+  };
+  load(0, x);
+  for (uint64_t k = 0; k < sa.L; k += 2 * U) {
+    load(k + U, y);
+    add(k, x);
+    load(k + 2 * U, x);
+    add(k + U, y);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // one lane per column (or per row for the generic case), sequential along the axis
 struct SeqScanArgs {
   RowIndexer<2> ix;   // dims enumerated by the lane: [0] input, [1] output strides
@@ -529,6 +767,121 @@ bool plan_cumsum(ScanShape& sh, const T* a, const T* c, int ndim, const size_t* 
 template <class T>
 bool chain_big(const ScanShape& sh) {
   return sh.p.L >= 2 * chain_te<T, kChainBigBlock, kChainBigVpt>();
+}
+
+// How a scan of a strided axis with unit-stride columns runs.
+struct ColScanRoute {
+  enum : int { kNone = 0, kLane = 1, kTiles = 2 };
+  int kind = kNone;
+  uint32_t cols = 0;                       // lane route: lanes
+  uint32_t strips = 0, groups = 0, tiles = 0, per = 0;  // per: groups per tile row of the grid
+  bool claim = false;
+  uint64_t words = 0;                      // tile route: status words (0 for a single tile)
+};
+// 16 lanes across (256-byte runs) by 512 lanes of 8 rows: 256-row tiles.  The few strips of a
+// narrow array cannot keep the 8 XCDs equally busy under the block numbering above, so below 32
+// strips, where their count is not a multiple of 8, tiles are claimed from a counter instead (their
+// predecessors are then running or finished on whatever XCD), in 512-row tiles of 1024 lanes, which
+// halve the look-backs.
+// Fewer columns than a 16-byte vector holds take 4 lanes across, one column each.
+constexpr int kColLpc = 16, kColLpcThin = 4, kColBlock = 512, kColBlockClaim = 1024, kColRpl = 8;
+constexpr uint64_t kColClaimGroups = 32;
+// One lane per column, which keeps the order of the reference, for axes of 64 to 384 rows ((300,
+// 20000) f32 26.8 -> 13.9 us with 32 rows of loads in flight twice over; (380, 500) 28.4 -> 14.1;
+// shorter axes are level with k_scan_seq) and, with 16 rows, for rows of 512 KB and more ((1000,
+// 131072) f32 229 -> 184 us, 210 in tiles; (1000, 65536) f64 203 -> 184, 209 in tiles).  From 1 MB
+// on k_scan_seq has enough lanes to itself: (1000, 262144) f32 369 us, 411 with 16 rows of loads.
+constexpr uint64_t kLaneScanRows = 64, kOrderedScanRows = 384;
+constexpr uint64_t kLaneScanBytes = uint64_t(512) << 10, kSeqScanBytes = uint64_t(1) << 20;
+
+template <class T>
+ColScanRoute col_scan_route(const ScanPlan& p) {
+  ColScanRoute r;
+  constexpr uint64_t VE = 16 / sizeof(T);
+  const uint64_t C = p.oshape[p.ond - 1];
+  if (p.kind != kColScan || C >= (uint64_t(1) << 31) || p.L >= (uint64_t(1) << 40)) return r;
+  const uint64_t outer = p.rows / C;
+  if (p.rows >= (uint64_t(1) << 31)) return r;
+  r.cols = uint32_t(p.rows);
+  const uint64_t row_bytes = p.rows * sizeof(T);
+  if (p.L < kLaneScanRows || row_bytes >= kSeqScanBytes) return r;
+  r.kind = ColScanRoute::kLane;
+  if (p.L <= kOrderedScanRows || row_bytes >= kLaneScanBytes) return r;
+  const bool thin = C < VE;
+  const uint64_t SC = thin ? kColLpcThin : kColLpc * VE;
+  const uint64_t strips = (C + SC - 1) / SC;
+  const uint64_t groups = outer * strips;
+  const bool claim = thin || (groups < kColClaimGroups && groups % 8 != 0);
+  const uint64_t TR = uint64_t(claim ? kColBlockClaim : kColBlock) / (thin ? kColLpcThin : kColLpc) * kColRpl;
+  const uint64_t tiles = (p.L + TR - 1) / TR;
+  const uint64_t per = claim ? groups : (groups + 7) / 8 * 8;
+  if (per * tiles >= (uint64_t(1) << 31)) return r;
+  r.kind = ColScanRoute::kTiles;
+  r.strips = uint32_t(strips);
+  r.groups = uint32_t(groups);
+  r.tiles = uint32_t(tiles);
+  r.per = uint32_t(per);
+  r.claim = claim;
+  r.words = tiles > 1 || claim ? (claim ? 1 : 0) + groups * tiles * SC * (sizeof(typename ScanAcc<T>::A) == 4 ? 1 : 2) : 0;
+  return r;
+}
+
+template <class T>
+void launch_scan_columns(const T* a, T* c, const ScanPlan& p, const ColScanRoute& r, uint64_t* status, uint32_t* fault,
+                         bool clear_fault, hipStream_t st) {
+  constexpr int VE = int(16 / sizeof(T));
+  ColScanArgs sa{};
+  sa.ix.nd = p.ond - 1;
+  for (int i = 0; i < sa.ix.nd; ++i) {
+    const int d = p.ond - 2 - i;
+    sa.ix.div[i] = make_fastdiv(uint32_t(p.oshape[d]));
+    sa.ix.stride[0][i] = p.istride[d];
+    sa.ix.stride[1][i] = p.ostride[d];
+  }
+  sa.L = p.L;
+  sa.C = p.oshape[p.ond - 1];
+  sa.ls_in = p.ls_in;
+  sa.ls_out = p.ls_out;
+  const uint64_t bytes = p.rows * p.L * sizeof(T);
+  sa.nt_load = bytes >= kStreamLoadBytes;
+  const bool nts = bytes >= kStreamStoreBytes;
+  if (r.kind == ColScanRoute::kLane) {
+    const unsigned grid = (r.cols + kSBlock - 1) / kSBlock;
+    const FastDiv cdiv = make_fastdiv(uint32_t(sa.C));
+    with_store_policy(nts, [&](auto NT) {
+      if (p.L <= kOrderedScanRows && p.rows * sizeof(T) < kLaneScanBytes)
+        k_scan_lane<T, 32, NT.value><<<grid, kSBlock, 0, st>>>(a, c, sa, cdiv, r.cols);
+      else
+        k_scan_lane<T, 16, NT.value><<<grid, kSBlock, 0, st>>>(a, c, sa, cdiv, r.cols);
+    });
+    return;
+  }
+  sa.gdiv = make_fastdiv(r.per);
+  sa.sdiv = make_fastdiv(r.strips);
+  sa.groups = r.groups;
+  sa.tiles = r.tiles;
+  sa.counter = r.claim ? reinterpret_cast<uint32_t*>(status) : nullptr;
+  sa.status = status + (r.claim ? 1 : 0);
+  sa.fault = fault;
+  sa.spin_limit = wait_spin_limit();
+  if (r.words) {
+    const unsigned cg = unsigned(r.words < 65536 * 256 ? (r.words + 255) / 256 : 65536);
+    k_scan_clear<<<cg, 256, 0, st>>>(status, r.words, clear_fault ? fault : nullptr);
+  }
+  // Rows off 128-byte lines leave each run's end lines half written: default stores let the L2 of
+  // the XCD that takes the neighbouring strip complete them.
+  const bool lines = (uint64_t(sa.ls_out) * sizeof(T)) % 128 == 0 && (reinterpret_cast<uintptr_t>(c) & 127) == 0;
+  with_store_policy(nts && lines, [&](auto NT) {
+    if (sa.C < VE)
+      k_scan_cols<T, 1, kColBlockClaim, kColRpl, kColLpcThin, true, NT.value>
+          <<<dim3(r.per * r.tiles), kColBlockClaim, 0, st>>>(a, c, sa);
+    else if (r.claim)
+      k_scan_cols<T, VE, kColBlockClaim, kColRpl, kColLpc, true, NT.value>
+          <<<dim3(r.per * r.tiles), kColBlockClaim, 0, st>>>(a, c, sa);
+    else
+      k_scan_cols<T, VE, kColBlock, kColRpl, kColLpc, false, NT.value>
+          <<<dim3(r.per * r.tiles), kColBlock, 0, st>>>(a, c, sa);
+  });
 }
 
 // tiles of the chained scan per row, 0 when the call does not take it
@@ -644,6 +997,14 @@ bool run_cumsum(const T* a, T* c, const ScanShape& sh, const ScanScratch& sc, hi
     k_scan_lookback<T><<<dim3(unsigned(uint64_t(p.rows) * tiles)), kLbBlock, 0, st>>>(a, c, sa);
     return true;
   }
+  if (const ColScanRoute r = col_scan_route<T>(p); r.kind != ColScanRoute::kNone) {
+    ColScanRoute q = r;
+    // a scratch too small for the status words: one lane per column vector
+    if (q.words != 0 && (sc.lb == nullptr || sc.fault == nullptr || q.words * 8 > sc.lb_bytes))
+      q.kind = ColScanRoute::kLane;
+    launch_scan_columns<T>(a, c, p, q, sc.lb, sc.fault, sc.clear_fault, st);
+    return true;
+  }
   SeqScanArgs sq{};
   sq.L = p.L;
   sq.ls_in = p.ls_in;
@@ -714,11 +1075,48 @@ int launch_cumsum_ws(const T* a, T* c, void* tmp, size_t tmp_bytes, int ndim, co
   return run_cumsum<T>(a, c, sh, sc, st) ? 0 : -1;
 }
 
+// Bytes of `tmp` with which musapy_cumsum_ws_v2 takes its fastest path for this call, given a
+// workspace of `ws_bytes`.
+template <class T>
+size_t cumsum_scratch(int ndim, const size_t* shape, const ssize_t* strides, int axis, size_t axis_len,
+                      size_t out_size, size_t ws_bytes) {
+  if (out_size == 0 || axis_len == 0 || ndim < 1 || ndim > kMaxDims || axis < 0 || axis >= ndim) return 0;
+  ScanShape sh;
+  plan_scan(sh.p, ndim, shape, strides, axis);
+  const uint64_t W = sizeof(typename ScanAcc<T>::A) == 4 ? 1 : 2;
+  if (sh.p.kind == kRowScan) {
+    if (sh.p.L <= 16) return 0;
+    if (const uint64_t ct = chain_tiles<T>(sh)) {
+      const uint64_t bytes = uint64_t(sh.p.rows) * ct * W * 8;
+      return bytes + 16 <= ws_bytes ? 0 : bytes;
+    }
+    constexpr uint64_t TE = uint64_t(kLbBlock) * kVpt * (16 / sizeof(T));
+    const uint64_t tiles = (sh.p.L + TE - 1) / TE;
+    return tiles > 1 ? (1 + uint64_t(sh.p.rows) * tiles * 2 * W) * 8 : 0;
+  }
+  const ColScanRoute r = col_scan_route<T>(sh.p);
+  return r.kind == ColScanRoute::kTiles ? r.words * 8 : 0;
+}
+
 }  // namespace mpy
 
 using namespace mpy;
 
 extern "C" {
+
+size_t musapy_cumsum_scratch_v1(int dtype, int ndim, const size_t* in_shape, const ssize_t* in_strides, int axis,
+                                size_t axis_len, size_t out_size, size_t workspace_bytes) {
+  switch (dtype) {
+    case MUSAPY_DT_I64:
+      return cumsum_scratch<int64_t>(ndim, in_shape, in_strides, axis, axis_len, out_size, workspace_bytes);
+    case MUSAPY_DT_F32:
+      return cumsum_scratch<float>(ndim, in_shape, in_strides, axis, axis_len, out_size, workspace_bytes);
+    case MUSAPY_DT_F64:
+      return cumsum_scratch<double>(ndim, in_shape, in_strides, axis, axis_len, out_size, workspace_bytes);
+    default:
+      return 0;
+  }
+}
 
 // rust/musapy-ops/src/kernels.rs:185-187
 void musapy_cumsum_i64_v3(const int64_t* a, int64_t* c, int64_t* tmp, int ndim, const size_t* in_shape,

@@ -857,25 +857,19 @@ Array cumsum_op(const Array& a, std::optional<size_t> axis, const Array* out) {
     if (bpr > 65536)
       throw ShapeError("cumsum: axis_len " + std::to_string(axis_len) +
                        " exceeds max supported length 16777216 (256^3)");
-    const size_t rows = out_size / std::max<size_t>(axis_len, 1);
     const int nd = int(kshape.size());
-    s->note_bounded_wait();  // row scans split into tiles wait on their predecessors
+    s->note_bounded_wait();  // scans split into tiles wait on their predecessors
     // Every cumsum reports its waits to the stream's workspace.  Many rows: the chained scan on
-    // that zeroed workspace (no scratch, no clear launch); fewer rows of several tiles: the
-    // look-back, on scratch of the reference's size (op_builder.rs:3315-3321), taken only when
-    // the first call reports that the path needs it.
+    // that zeroed workspace (no scratch, no clear launch); fewer rows of several tiles, and long
+    // strided axes: a look-back on scratch.
     const int dt = ct == Dtype::Int64 ? MUSAPY_DT_I64 : ct == Dtype::Float32 ? MUSAPY_DT_F32 : MUSAPY_DT_F64;
     void* ws = s->reduce_workspace();
+    const size_t scratch = musapy_cumsum_scratch_v1(dt, nd, kshape.data(), kstrides.data(), kaxis, axis_len, out_size,
+                                                    Stream::kReduceWorkspaceBytes);
     BufferRef tmp;
-    if (musapy_cumsum_ws_v2(dt, aw->data_ptr(), r.data_ptr(), nullptr, 0, nd, kshape.data(), kstrides.data(), kaxis,
-                            axis_len, out_size, ws, Stream::kReduceWorkspaceBytes, s->raw()) != 0) {
-      (void)musapy_kernels_take_error();  // 1: the path needs scratch (any other error recurs below)
-      const size_t scratch = (bpr > 256 ? rows * (bpr + (bpr + 255) / 256) : rows * bpr) * element_size(ct);
-      tmp = Buffer::alloc(std::max<size_t>(scratch, 8), a.device, s);
-      (void)musapy_cumsum_ws_v2(dt, aw->data_ptr(), r.data_ptr(), tmp->ptr(), tmp->nbytes(), nd, kshape.data(),
-                                kstrides.data(), kaxis, axis_len, out_size, ws, Stream::kReduceWorkspaceBytes,
-                                s->raw());
-    }
+    if (scratch > 0) tmp = Buffer::alloc(scratch, a.device, s);
+    (void)musapy_cumsum_ws_v2(dt, aw->data_ptr(), r.data_ptr(), tmp ? tmp->ptr() : nullptr, scratch, nd, kshape.data(),
+                              kstrides.data(), kaxis, axis_len, out_size, ws, Stream::kReduceWorkspaceBytes, s->raw());
     check_launch("cumsum");
   }
   aw->data->record_read(s);

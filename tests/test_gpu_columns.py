@@ -93,3 +93,48 @@ def test_column_results_repeat():
         ms.max(X, axis=(0, 1))
         assert_bits_equal(ms.argmax(X, axis=0).numpy(), first[1], "argmax")
     assert_bits_equal(first[1], R.reduce(x, "argmax", 0), "argmax against the oracle")
+
+
+# ---- cumsum down the columns ----
+SCAN_SHAPES = [
+    ((63, 5), 0), ((64, 3), 0), ((384, 70), 0),                    # sequential, one lane per column
+    ((385, 64), 0), ((511, 65), 0), ((513, 3), 0),                 # one tile; two; fewer columns than a vector
+    ((2049, 1), 0), ((3000, 2), 0), ((2600, 7), 0),                # thin arrays, claimed tiles
+    ((1025, 513), 0), ((700, 1030), 0), ((2305, 130), 0),          # strips: a multiple of 8 or not, ragged
+    ((3, 900, 33), 1), ((2, 3, 600, 18), 2), ((9, 400, 66), 1),    # outer dims
+]
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64, np.int64])
+def test_column_scan_shapes(dt):
+    tol = {np.float32: 1e-5, np.float64: 1e-12}.get(dt)
+    for shape, axis in SCAN_SHAPES:
+        x = values("sum", dt, shape)
+        got = ms.cumsum(dev(x), axis=axis).numpy()
+        want = R.cumsum(x, axis)
+        what = f"cumsum {np.dtype(dt).name} {shape} axis {axis}"
+        if tol is None or shape[axis] <= 384:  # short axes keep the order of the reference
+            assert_bits_equal(got, want, what)
+        else:
+            assert np.all(np.abs(got - want) <= tol * np.cumsum(np.abs(x.astype(np.float64)), axis=axis)), what
+        for _ in range(2):
+            assert_bits_equal(ms.cumsum(dev(x), axis=axis).numpy(), got, what + " again")
+
+
+def test_column_scan_views_and_specials():
+    base = RNG.integers(-100, 100, (1500, 90)).astype(np.int64)
+    B = dev(base)
+    assert_bits_equal(ms.cumsum(ms.flip(B, 0), axis=0).numpy(), np.cumsum(base[::-1], 0), "reversed axis")
+    assert_bits_equal(ms.cumsum(ms.slice(B, [(1, 1500, 2), (3, 88, 1)]), axis=0).numpy(),
+                      np.cumsum(base[1:1500:2, 3:88], 0), "every second row of some columns")
+    for dt in (np.float32, np.float64):
+        x = RNG.random((1300, 40)).astype(dt)
+        x[700, 3] = np.inf
+        x[900, 4] = np.nan
+        x[10, 5], x[1200, 5] = np.inf, -np.inf
+        x[:, 6] = -0.0
+        got, want = ms.cumsum(dev(x), axis=0).numpy(), R.cumsum(x, 0)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+        ok = np.isfinite(want)
+        assert np.all(np.abs(got[ok] - want[ok]) <= 1e-5 * want[ok])
+        assert not np.signbit(got[:, 6]).any()

@@ -128,6 +128,17 @@ def test_row_scan_look_back_gives_up_and_recovers():
     _fresh_stream_case(lambda: (ms.from_numpy(y),), lambda Y: ms.cumsum(Y, axis=1), check)
 
 
+@pytest.mark.parametrize("shape", [(4000, 40), (4000, 1000)])  # claimed tiles, numbered tiles
+def test_column_scan_gives_up_and_recovers(shape):
+    y = RNG.random(shape)
+    want = R.cumsum(y, 0)
+
+    def check(got, what):
+        assert np.all(np.abs(got - want) <= 1e-12 * np.abs(want)), what
+
+    _fresh_stream_case(lambda: (ms.from_numpy(y),), lambda Y: ms.cumsum(Y, axis=0), check)
+
+
 def test_chained_row_scan_gives_up_and_recovers():
     y = RNG.random((520, 20_000))
     want = R.cumsum(y, 1)
