@@ -346,6 +346,16 @@ enum { MUSAPY_RED_SUM = 0, MUSAPY_RED_PROD, MUSAPY_RED_MAX, MUSAPY_RED_MIN, MUSA
        MUSAPY_RED_ARGMIN };
 int musapy_reduce_fused_v1(int op, int dtype, const void* a, void* c, int ndim, const size_t* in_shape, const ssize_t* in_strides, int axis, size_t axis_len, size_t out_size, size_t tiles, void* workspace, size_t workspace_bytes, hipStream_t stream);
 
+/* ---- reductions of narrow integers without a cast (new; no counterpart in kernels.rs) ----
+ * `op` over an integer array `a` of `src_dtype`, with the result the reference gets by casting the
+ * array first (op_builder.rs:2209-2225): int64 values for SUM, PROD, MAX and MIN, int64 indices for
+ * ARGMAX and ARGMIN, float64 for MEAN.  8-, 16- and 32-bit sources take every op, 64-bit ones only
+ * MEAN.  `tmp` holds the partials of a call that is split into tiles: musapy_reduce_int_scratch_v1
+ * bytes, arbitrary contents; NULL or less runs in one launch.  Returns 0 when launched, -1 when not
+ * covered (nothing launched: cast, then reduce; extents of 2^31 and more, empty reductions). */
+size_t musapy_reduce_int_scratch_v1(int op, int src_dtype, int ndim, const size_t* in_shape, const ssize_t* in_strides, int axis, size_t axis_len, size_t out_size);
+int musapy_reduce_int_v1(int op, int src_dtype, const void* a, void* c, int ndim, const size_t* in_shape, const ssize_t* in_strides, int axis, size_t axis_len, size_t out_size, void* tmp, size_t tmp_bytes, hipStream_t stream);
+
 /* ---- cumsum on a zeroed workspace (new; no counterpart in kernels.rs) ----
  * The chained scan of musapy_cumsum_*_v3 for many (>= 512) unit-stride rows of several tiles,
  * with its per-tile prefixes in `workspace` instead of the reference's scratch `tmp`: the

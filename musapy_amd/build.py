@@ -37,6 +37,7 @@ CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function"]
 HIP_SOURCES = [
     "kernels/elementwise.hip",
     "kernels/reduce.hip",
+    "kernels/reduce_int.hip",
     "kernels/scan.hip",
     "runtime/hip_runtime.cpp",
 ]

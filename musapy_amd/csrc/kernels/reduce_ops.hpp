@@ -195,14 +195,18 @@ template <class T> __device__ inline T ext_none();  // value written for an empt
 template <> __device__ inline float ext_none<float>() { return qnan<float>(); }
 template <> __device__ inline double ext_none<double>() { return qnan<double>(); }
 template <> __device__ inline int64_t ext_none<int64_t>() { return INT64_MIN; }  // never kept by '>'
+template <> __device__ inline int32_t ext_none<int32_t>() { return INT32_MIN; }
 template <class T> __device__ inline T ext_none_min();
 template <> __device__ inline float ext_none_min<float>() { return qnan<float>(); }
 template <> __device__ inline double ext_none_min<double>() { return qnan<double>(); }
 template <> __device__ inline int64_t ext_none_min<int64_t>() { return INT64_MAX; }
 
+template <> __device__ inline int32_t ext_none_min<int32_t>() { return INT32_MAX; }
+
 // ---------------------------------------------------------------------------------------------
 // conversions of an accumulator to the values written out
 template <class T, class A> __device__ inline T narrow(A a) { return T(a); }
+template <> __device__ inline double narrow<double, uint64_t>(uint64_t a) { return double(int64_t(a)); }
 template <> __device__ inline int64_t narrow<int64_t, uint64_t>(uint64_t a) { return int64_t(a); }
 template <> __device__ inline c64 narrow<c64, c128>(c128 a) { return c64{float(a.re), float(a.im)}; }
 template <> __device__ inline c128 narrow<c128, c128>(c128 a) { return a; }
@@ -210,6 +214,8 @@ template <> __device__ inline c128 narrow<c128, c128>(c128 a) { return a; }
 // mean = sum / count where count is the reference's repeated "+1" in T (exact until 2^24 for
 // f32, 2^53 for f64, constant afterwards); complex means divide re and im by the f64 length.
 template <class T, class A> __device__ inline T mean_of(A s, double count) { return T(s / A(count)); }
+// the exact sum of integers of at most 32 bits
+template <> __device__ inline double mean_of<double, uint64_t>(uint64_t s, double count) { return double(int64_t(s)) / count; }
 template <> __device__ inline c64 mean_of<c64, c128>(c128 s, double n) { return c64{float(s.re / n), float(s.im / n)}; }
 template <> __device__ inline c128 mean_of<c128, c128>(c128 s, double n) { return c128{s.re / n, s.im / n}; }
 

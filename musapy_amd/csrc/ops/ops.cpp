@@ -552,20 +552,21 @@ void red_single(ReduceKernel k, Dtype ct, const RedCall& c, void* out) {
 #undef R1
 }
 
+int red_op(ReduceKernel k) {
+  switch (k) {
+    case ReduceKernel::Sum: return MUSAPY_RED_SUM;
+    case ReduceKernel::Prod: return MUSAPY_RED_PROD;
+    case ReduceKernel::Max: return MUSAPY_RED_MAX;
+    case ReduceKernel::Min: return MUSAPY_RED_MIN;
+    case ReduceKernel::Mean: return MUSAPY_RED_MEAN;
+    case ReduceKernel::Argmax: return MUSAPY_RED_ARGMAX;
+    default: return MUSAPY_RED_ARGMIN;
+  }
+}
+
 // partial + final in one launch (musapy_reduce_fused_v1) with the stream's workspace; false when
 // the kernel library does not cover the case (then the two-stage path runs)
 bool red_fused(ReduceKernel k, Dtype ct, const RedCall& c, void* out, size_t tiles, Stream& s) {
-  int op = 0;
-  switch (k) {
-    case ReduceKernel::Sum: op = MUSAPY_RED_SUM; break;
-    case ReduceKernel::Prod: op = MUSAPY_RED_PROD; break;
-    case ReduceKernel::Max: op = MUSAPY_RED_MAX; break;
-    case ReduceKernel::Min: op = MUSAPY_RED_MIN; break;
-    case ReduceKernel::Mean: op = MUSAPY_RED_MEAN; break;
-    case ReduceKernel::Argmax: op = MUSAPY_RED_ARGMAX; break;
-    case ReduceKernel::Argmin: op = MUSAPY_RED_ARGMIN; break;
-    default: return false;
-  }
   int dt = 0;
   switch (ct) {
     case Dtype::Float32: dt = MUSAPY_DT_F32; break;
@@ -575,12 +576,15 @@ bool red_fused(ReduceKernel k, Dtype ct, const RedCall& c, void* out, size_t til
     case Dtype::Complex128: dt = MUSAPY_DT_C128; break;
     default: return false;
   }
-  if (musapy_reduce_fused_v1(op, dt, c.a, out, c.nd, c.shape, c.strides, c.axis, c.axis_len, c.out_size, tiles,
+  if (musapy_reduce_fused_v1(red_op(k), dt, c.a, out, c.nd, c.shape, c.strides, c.axis, c.axis_len, c.out_size, tiles,
                              s.reduce_workspace(), Stream::kReduceWorkspaceBytes, c.s) != 0)
     return false;
   s.note_bounded_wait();
   return true;
 }
+
+// integer dtypes, whose reduction starts with a cast in the reference (op_builder.rs:2209-2225)
+bool is_int(Dtype d) { return dtype_category(d) == 1 || dtype_category(d) == 2; }
 
 // partial -> final for value reductions (sum/prod/max/min/mean)
 void red_two_stage(ReduceKernel k, Dtype ct, const RedCall& c, void* out, size_t tiles, void* partials) {
@@ -688,8 +692,18 @@ Array reduction_axis(const Array& a, std::optional<size_t> axis, bool keepdims, 
   check_out(op, out, out_shape, out_dt, a, "expected output shape", "expected");
   StreamPtr s = pick_stream(a, out);
   std::optional<Array> cast;
-  if (a.dtype != ct) cast = cast_array(a, ct, s);
-  const Array* aw = cast ? &*cast : &a;
+  const Array* aw = &a;
+  // narrow integers are widened by the reduction itself; only what that does not cover is cast first
+  const bool direct = a.dtype != ct && is_int(a.dtype) && total > 0 && axis_len < (size_t(1) << 31) &&
+                      out_size < (size_t(1) << 31) && (element_size(a.dtype) < 8 || k == ReduceKernel::Mean);
+  if (a.dtype == Dtype::Uint64 && ct == Dtype::Int64) {
+    cast = a;  // the same bits
+    cast->dtype = ct;
+    aw = &*cast;
+  } else if (a.dtype != ct && !direct) {
+    cast = cast_array(a, ct, s);
+    aw = &*cast;
+  }
   Array r = make_output(out, out_shape, out_dt, a.device, s, {aw});
   aw->data->wait_last_write_on(s);
   std::optional<Array> flat;
@@ -705,6 +719,19 @@ Array reduction_axis(const Array& a, std::optional<size_t> axis, bool keepdims, 
     Strides kstrides = axis ? aw->layout.strides : Strides{1};
     RedCall c{aw->data_ptr(), int(kshape.size()), kshape.data(), kstrides.data(), kaxis, axis_len, out_size, s->raw()};
     const size_t es = element_size(ct);
+    if (direct) {
+      const size_t need = musapy_reduce_int_scratch_v1(red_op(k), int(aw->dtype), c.nd, c.shape, c.strides, c.axis,
+                                                       axis_len, out_size);
+      BufferRef tmp;
+      if (need > 0) tmp = Buffer::alloc(need, a.device, s);
+      if (musapy_reduce_int_v1(red_op(k), int(aw->dtype), c.a, r.data_ptr(), c.nd, c.shape, c.strides, c.axis, axis_len,
+                               out_size, tmp ? tmp->ptr() : nullptr, need, s->raw()) != 0)
+        throw KernelError(std::string(op) + ": integer reduction refused its arguments");
+      check_launch(op);
+      aw->data->record_read(s);
+      r.data->record_write(s);
+      return r;
+    }
     size_t tiles = axis_len == 0 ? 1
                                  : musapy_reduce_tiles_hint(c.nd, c.shape, c.strides, c.axis, axis_len, out_size, es);
     if (tiles <= 1) {
