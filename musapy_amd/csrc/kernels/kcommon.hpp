@@ -111,8 +111,10 @@ __device__ inline Vec<T, N> vload_nt(const T* p) {
 template <int B, int A> struct ElWord {
   typedef typename NtWord<B>::type type __attribute__((aligned(A)));
 };
-template <typename T, int N>
-__device__ inline Vec<T, N> vload_el(const T* p, bool nt) {
+// Streaming unless NT is false: a template parameter, since the compiler merges the two loads of a
+// runtime choice into one default load ((8192, 8192) f32 row sum 40.0 -> 44.6 us that way).
+template <typename T, int N, bool NT = true>
+__device__ inline Vec<T, N> vload_el(const T* p) {
   constexpr int kB = int(sizeof(T) * N);
   constexpr int kW = kB > 16 ? 16 : kB;
   constexpr int kA = int(alignof(T)) < kW ? int(alignof(T)) : kW;
@@ -122,7 +124,8 @@ __device__ inline Vec<T, N> vload_el(const T* p, bool nt) {
   W w[kB / kW];
 #pragma unroll
   for (int i = 0; i < kB / kW; ++i)
-    w[i] = nt ? __builtin_nontemporal_load(reinterpret_cast<const U*>(p) + i) : reinterpret_cast<const U*>(p)[i];
+    if constexpr (NT) w[i] = __builtin_nontemporal_load(reinterpret_cast<const U*>(p) + i);
+    else w[i] = reinterpret_cast<const U*>(p)[i];
   Vec<T, N> v;
   __builtin_memcpy(&v, w, kB);
   return v;

@@ -100,8 +100,10 @@ bool int_plan(ReducePlan& p, const IntCall& c) {
 template <class Op, class T, class S, class O, int WRITE>
 void launch_int_rows(const S* a, RedOut<O> out, const ReducePlan& p, size_t tiles, hipStream_t st) {
   constexpr int V = ivec<S>();
+  if constexpr (WRITE == kWriteFinal) {
+    if (tiles == 1 && launch_short<Op, T, V, S, O>(a, out, p, st)) return;
+  }
   RowArgs ra{};
-  ra.nt = true;
   ra.ix = out_indexer(p, p.ond);
   ra.R = p.R;
   ra.rs = p.rstride;

@@ -11,7 +11,8 @@
 //        rows, and LDS merges the waves -- every load is a coalesced row segment.  Narrow rows
 //        take whole rows per step instead (span kernel), and reductions with many outputs one
 //        lane per 16 bytes of them (lane kernel); col_route holds the lines between the three.
-// Large reductions are split into tiles: the partial entry points write [out_size][tiles] and
+// Reductions write next to nothing, so their loads stream at every volume measured (the 128 MB c64
+// sum: 5.1 TB/s, 4.6 with default loads).  Large reductions are split into tiles: the partial entry points write [out_size][tiles] and
 // the final entry points reduce those rows with the same row kernel.  Every combine order is
 // fixed, so results are identical from run to run.
 #pragma once
@@ -182,19 +183,22 @@ struct RowArgs {
   uint64_t chunk;     // axis elements per tile (multiple of VEC when VEC > 1)
   uint32_t tiles;
   uint64_t nwork;     // out_size * tiles
-  bool nt;            // streaming loads (launch input volume >= kStreamLoadBytes)
+  bool nt;            // streaming loads, where the kernel leaves the choice to run time
 };
 
 // One lane's share of a segment: lane l of a GROUP-lane group reduces elements l*VEC, l*VEC +
 // GROUP*VEC, ... of the n-element segment at tb (indices relative to tb).  tb is unit-stride with
-// VEC > 1 (any element address).  S: the stored element, widened to T as it is read.  Lane 0 also returns
+// VEC > 1 (any element address).  S: the stored element, widened to T as it is read.  WHOLE: n is a
+// multiple of a round (GROUP * VEC * UNROLL) and tb 16-byte aligned; the loads then keep the
+// runtime choice of policy, whose scalar branches between the loads leave argmax over the rows of
+// (8192, 8192) f32 at 39.9 us, against 41.2 us with the loads back to back.  Lane 0 also returns
 // the segment's first element in `first` (ordered reductions need it for the NaN-at-0 rule; it
 // is kept from the load instead of being read again at the end).  The fold continues `acc`, and
 // ordered reductions record indices as base + (index in the segment).
-template <class Op, class T, int GROUP, int VEC, int UNROLL, class S = T>
+template <class Op, class T, int GROUP, int VEC, int UNROLL, class S = T, bool WHOLE = false>
 __device__ inline typename Op::A accumulate_segment(const S* __restrict__ tb, uint32_t n, int l, int64_t rs,
-                                                    bool nt, T& first, typename Op::A acc = Op::init(),
-                                                    int64_t base = 0) {
+                                                    T& first, typename Op::A acc = Op::init(),
+                                                    int64_t base = 0, bool nt = true) {
   uint32_t k = uint32_t(l) * VEC;
   constexpr uint32_t stepk = uint32_t(GROUP) * VEC;
   const bool lead = l == 0;  // lane 0 starts at element 0
@@ -202,7 +206,10 @@ __device__ inline typename Op::A accumulate_segment(const S* __restrict__ tb, ui
     for (; k + (UNROLL - 1) * stepk + VEC <= n; k += UNROLL * stepk) {
       Vec<S, VEC> x[UNROLL];
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u) x[u] = vload_el<S, VEC>(tb + k + u * stepk, nt);
+      for (int u = 0; u < UNROLL; ++u) {
+        if constexpr (WHOLE) x[u] = vload_pol<S, VEC>(tb + k + u * stepk, nt);
+        else x[u] = vload_el<S, VEC>(tb + k + u * stepk);
+      }
       // all UNROLL loads are issued before the first use (the scheduler would otherwise hoist
       // arithmetic between them and wait on the first load early)
       __builtin_amdgcn_sched_barrier(0);
@@ -214,20 +221,38 @@ __device__ inline typename Op::A accumulate_segment(const S* __restrict__ tb, ui
       if (Op::kOrdered && lead && k == 0) first = xs[0][0];
       acc = Op::template step_chunk<UNROLL, VEC>(acc, xs, k, stepk, base);
     }
-    for (; k + VEC <= n; k += stepk) {  // whole vectors left
-      Vec<S, VEC> x = vload_el<S, VEC>(tb + k, nt);
-      if (Op::kOrdered && lead && k == 0) first = T(x.v[0]);
+    // The rest in one round of unconditional loads: a vector that the end of the segment cuts is
+    // read from where it still fits, and its elements below k (the vector's before) are skipped.
+    if (WHOLE) {
+    } else if (k < n && n >= uint32_t(VEC)) {
+      Vec<S, VEC> x[UNROLL];
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) acc = Op::step(acc, T(x.v[v]), base + int64_t(k + v));
-    }
-    if (k < n) {  // the last, partial vector of the tile
+      for (int u = 0; u < UNROLL; ++u) {
+        const uint32_t ku = k + u * stepk;
+        x[u] = vload_el<S, VEC>(tb + (ku + VEC <= n ? ku : n - VEC));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (Op::kOrdered && lead && k == 0) first = T(x[0].v[0]);
 #pragma unroll
-      for (int v = 0; v < VEC; ++v)
-        if (k + v < n) {
-          const T x = T(tb[k + v]);
-          if (Op::kOrdered && lead && k + v == 0) first = x;
-          acc = Op::step(acc, x, base + int64_t(k + v));
+      for (int u = 0; u < UNROLL; ++u) {
+        const uint32_t ku = k + u * stepk;
+        if (ku + VEC <= n) {
+          T xs[1][VEC];
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) xs[0][v] = T(x[u].v[v]);
+          acc = Op::template step_chunk<1, VEC>(acc, xs, ku, 0, base);
+        } else if (ku < n) {
+#pragma unroll
+          for (int v = 0; v < VEC; ++v)
+            if (n - VEC + v >= ku) acc = Op::step(acc, T(x[u].v[v]), base + int64_t(n - VEC + v));
         }
+      }
+    } else {
+      for (; k < n; ++k) {  // fewer elements than a vector (lane 0)
+        const T x = T(tb[k]);
+        if (Op::kOrdered && lead && k == 0) first = x;
+        acc = Op::step(acc, x, base + int64_t(k));
+      }
     }
   } else {
     for (; k + (UNROLL - 1) * stepk < n; k += UNROLL * stepk) {
@@ -247,7 +272,7 @@ __device__ inline typename Op::A accumulate_segment(const S* __restrict__ tb, ui
   return acc;
 }
 
-template <class Op, class T, int BS, int GROUP, int VEC, int UNROLL, int WRITE, class S = T, class O = T>
+template <class Op, class T, int BS, int GROUP, int VEC, int UNROLL, int WRITE, class S = T, class O = T, bool WHOLE = false>
 __global__ __launch_bounds__(BS) void k_reduce_row(const S* __restrict__ a, RowArgs ra, RedOut<O> out) {
   using A = typename Op::A;
   constexpr int kPer = BS / GROUP;  // items per block
@@ -272,7 +297,7 @@ __global__ __launch_bounds__(BS) void k_reduce_row(const S* __restrict__ a, RowA
     const uint64_t k1 = k0 + ra.chunk < ra.R ? k0 + ra.chunk : ra.R;
     const S* tb = a + off[0] + int64_t(k0) * ra.rs;  // indices below are relative to the tile start
     const uint32_t n = k1 > k0 ? uint32_t(k1 - k0) : 0u;
-    acc = accumulate_segment<Op, T, GROUP, VEC, UNROLL, S>(tb, n, l, ra.rs, ra.nt, first);
+    acc = accumulate_segment<Op, T, GROUP, VEC, UNROLL, S, WHOLE>(tb, n, l, ra.rs, first, Op::init(), 0, ra.nt);
   }
   acc = group_reduce<Op, GROUP>(acc);
   if (live && (GROUP <= kWave ? l == 0 : threadIdx.x == 0)) {
@@ -369,7 +394,7 @@ __global__ __launch_bounds__(kRowBS) void k_reduce_row_fused(const T* __restrict
     const uint32_t n = k1 > k0 ? uint32_t(k1 - k0) : 0u;
     T first{};
     A acc = accumulate_segment<Op, T, kRowBS, VEC, UNROLL>(a + off[0] + int64_t(k0) * ra.rs, n, threadIdx.x, ra.rs,
-                                                           ra.nt, first);
+                                                           first);
     acc = group_reduce<Op, kRowBS>(acc);
     if (threadIdx.x == 0) {
       if (t == 0 && ra.R > 0) acc = absorb_first<Op, T>(acc, first);
@@ -495,7 +520,7 @@ __device__ inline typename OpF::A all_stream(const T* __restrict__ a, uint64_t n
   if (c == whole && whole * kChunk < n) {  // the last, partial chunk
     T f{};
     acc = accumulate_segment<OpF, T, BS, VEC, UNROLL>(a + c * kChunk, uint32_t(n - c * kChunk), threadIdx.x, 1,
-                                                      true, f, acc, int64_t(c * kChunk));
+                                                      f, acc, int64_t(c * kChunk));
     if (c == 0) first = f;
   }
   return acc;
@@ -659,7 +684,6 @@ struct ColArgs {
   int64_t rs;
   uint64_t chunk;
   uint32_t tiles;
-  bool nt;            // streaming loads
 };
 
 // A lane's first column.  The last vector of a row of odd length is moved back to end with the row
@@ -697,7 +721,7 @@ __device__ inline void col_partial(const T* __restrict__ a, const ColArgs& ca, u
       // the axis's row 0 for the NaN-at-0 rule: one extra load by wave 0 of tile 0, kept out of
       // the streaming loop (a capture inside it cost the ordered kernels ~10% on (8192, 8192))
       if (Op::kOrdered && k == 0 && k < k1) {
-        const Vec<T, VEC> x = vload_el<T, VEC>(base, ca.nt);
+        const Vec<T, VEC> x = vload_el<T, VEC>(base);
 #pragma unroll
         for (int v = 0; v < VEC; ++v) first[v] = x.v[v];
       }
@@ -712,7 +736,7 @@ __device__ inline void col_partial(const T* __restrict__ a, const ColArgs& ca, u
       Vec<T, VEC> x[UNROLL], y[UNROLL];  // ping-pong buffers
       auto load = [&](uint64_t kk, Vec<T, VEC>(&d)[UNROLL]) {
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u) d[u] = vload_el<T, VEC>(base + int64_t(kk + u * kWaves) * ca.rs, ca.nt);
+        for (int u = 0; u < UNROLL; ++u) d[u] = vload_el<T, VEC>(base + int64_t(kk + u * kWaves) * ca.rs);
       };
       auto fold = [&](uint64_t kk, const Vec<T, VEC>(&src)[UNROLL]) {
 #pragma unroll
@@ -750,7 +774,7 @@ __device__ inline void col_partial(const T* __restrict__ a, const ColArgs& ca, u
         }
       }
       for (; k < k1; k += kWaves) {
-        Vec<T, VEC> x = vload_el<T, VEC>(base + int64_t(k) * ca.rs, ca.nt);
+        Vec<T, VEC> x = vload_el<T, VEC>(base + int64_t(k) * ca.rs);
 #pragma unroll
         for (int v = 0; v < VEC; ++v) acc[v] = Op::step(acc[v], x.v[v], int64_t(k - k0));
       }
@@ -866,7 +890,7 @@ __global__ __launch_bounds__(kSpanBS) void k_reduce_span(const S* __restrict__ a
     auto load = [&](uint64_t k, Vec<S, VEC>(&d)[UNROLL]) {
       const S* q = lp + int64_t((uint64_t(t) + k * sa.tiles) * step_rows) * sa.rs;
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u) d[u] = vload_el<S, VEC>(q + int64_t(uint64_t(u) * sa.m) * sa.rs, true);
+      for (int u = 0; u < UNROLL; ++u) d[u] = vload_el<S, VEC>(q + int64_t(uint64_t(u) * sa.m) * sa.rs);
     };
     auto fold = [&](uint64_t k, const Vec<S, VEC>(&src)[UNROLL]) {
       const uint32_t row = uint32_t((uint64_t(t) + k * sa.tiles) * step_rows);
@@ -890,7 +914,7 @@ __global__ __launch_bounds__(kSpanBS) void k_reduce_span(const S* __restrict__ a
       for (int u = 0; u < UNROLL; ++u) {
         const uint64_t row = base + uint64_t(u) * sa.m;
         const S* q = row + rv[VEC - 1] < sa.R ? lp + int64_t(row) * sa.rs : safe;
-        x[u] = vload_el<S, VEC>(q, true);
+        x[u] = vload_el<S, VEC>(q);
       }
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
@@ -1016,7 +1040,7 @@ __global__ __launch_bounds__(kRBlock) void k_reduce_lane(const S* __restrict__ a
     first[v] = T{};
   }
   if constexpr (Op::kOrdered) {
-    const Vec<S, VEC> x = vload_el<S, VEC>(p, true);
+    const Vec<S, VEC> x = vload_el<S, VEC>(p);
 #pragma unroll
     for (int v = 0; v < VEC; ++v) first[v] = T(x.v[v]);
   }
@@ -1024,7 +1048,7 @@ __global__ __launch_bounds__(kRBlock) void k_reduce_lane(const S* __restrict__ a
   for (; k + UNROLL <= R; k += UNROLL) {
     Vec<S, VEC> x[UNROLL];
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) x[u] = vload_el<S, VEC>(p + int64_t(k + u) * rs, true);
+    for (int u = 0; u < UNROLL; ++u) x[u] = vload_el<S, VEC>(p + int64_t(k + u) * rs);
 #pragma unroll
     for (int v = 0; v < VEC; ++v) {
       T xs[UNROLL][1];
@@ -1034,7 +1058,7 @@ __global__ __launch_bounds__(kRBlock) void k_reduce_lane(const S* __restrict__ a
     }
   }
   for (; k < R; ++k) {
-    const Vec<S, VEC> x = vload_el<S, VEC>(p + int64_t(k) * rs, true);
+    const Vec<S, VEC> x = vload_el<S, VEC>(p + int64_t(k) * rs);
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] = Op::step(acc[v], T(x.v[v]), int64_t(k));
   }
@@ -1728,6 +1752,89 @@ inline size_t tiles_hint(const ReducePlan& p, size_t es) {
   return size_t(tiles < 1 ? 1 : tiles);
 }
 
+// --------------------------------------------------------------------------------------------
+// Short unit-stride rows (at most 128 vectors), many of them: GROUP lanes per row, U rows per group in flight,
+// neighbouring groups on neighbouring rows.  The vector that the end of a row cuts is read from
+// where it still fits and its elements that belong to the vector before are skipped, so every load
+// is a whole 16 bytes.  Against the group kernels with one row each: (300000, 101) f32 sum 70.4 ->
+// 20.9 us (5.8 TB/s), (1000000, 33) 54.2 -> 26.2, (3000000, 8) 124.3 -> 19.4, (1000000, 17) f64 64.2
+// -> 30.5; max of (1000000, 33) 76.3 -> 40.9, where the compares of each element begin to bind.
+template <class Op, class T, int GROUP, int VEC, int U, class S = T, class O = T>
+__global__ __launch_bounds__(kRBlock) void k_reduce_short(const S* __restrict__ a, RowIndexer<1> ix, uint32_t R,
+                                                          uint32_t rows, RedOut<O> out) {
+  using A = typename Op::A;
+  constexpr uint32_t kGroups = kRBlock / GROUP;
+  const uint32_t l = threadIdx.x % GROUP;
+  const uint32_t row0 = blockIdx.x * (kGroups * U) + threadIdx.x / GROUP;
+  const S* p[U];
+  A acc[U];
+  T first[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const uint32_t row = row0 + u * kGroups < rows ? row0 + u * kGroups : rows - 1;
+    int64_t off[1];
+    row_offsets<1>(ix, row, off);
+    p[u] = a + off[0];
+    acc[u] = Op::init();
+    first[u] = T{};
+  }
+  for (uint32_t k = l * VEC; k < R; k += GROUP * VEC) {
+    const uint32_t kk = k + VEC <= R ? k : R - VEC;
+    Vec<S, VEC> x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) x[u] = vload_el<S, VEC>(p[u] + kk);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (Op::kOrdered && k == 0) first[u] = T(x[u].v[0]);
+#pragma unroll
+      for (int v = 0; v < VEC; ++v)
+        if (kk + v >= k) acc[u] = Op::step(acc[u], T(x[u].v[v]), int64_t(kk + v));
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    A r = group_reduce<Op, GROUP>(acc[u]);
+    const uint32_t row = row0 + u * kGroups;
+    if (l == 0 && row < rows) write_result<Op, T, kWriteFinal, O>(out, row, absorb_first<Op, T>(r, first[u]), 0);
+  }
+}
+
+// Lanes per row: enough for the row in one step (two from 65 vectors on).  Fewer lanes walking more
+// steps each spread a load instruction over more lines: (300000, 101) f32 sum 20.9 us with 32 lanes,
+// 28.4 with up to 2 steps, 38.4 with up to 4; (3000000, 8) 19.4 us with 2 lanes, 31.9 with 1.
+inline int short_group(uint64_t vecs) {
+  int g = 1;
+  while (g < kWave && uint64_t(g) < vecs) g *= 2;
+  return g;
+}
+template <class Op, class T, int VEC, class S, class O>
+bool launch_short(const S* a, RedOut<O> out, const ReducePlan& p, hipStream_t st) {
+  const uint64_t vecs = ceil_div(p.R, uint64_t(VEC));
+  if (p.rstride != 1 || p.R < uint64_t(VEC) || vecs > 2 * kWave || p.out_size >= (uint64_t(1) << 31)) return false;
+  constexpr int U = sizeof(typename Op::A) <= 8 ? 4 : 2;
+  const int g = short_group(vecs);
+  // below two blocks per CU the rows in flight per group leave the GPU idle: (256, 256) f32 argmax
+  // 4.4 us, against 3.7 with a wave per row
+  if (ceil_div(p.out_size, uint64_t(kRBlock / g) * U) < 512) return false;
+  const RowIndexer<1> ix = out_indexer(p, p.ond);
+  const uint32_t R = uint32_t(p.R), rows = uint32_t(p.out_size);
+  auto go = [&](auto G) {
+    constexpr int kG = decltype(G)::value;
+    const unsigned grid = unsigned(ceil_div(rows, uint64_t(kRBlock / kG) * U));
+    k_reduce_short<Op, T, kG, VEC, U, S, O><<<grid, kRBlock, 0, st>>>(a, ix, R, rows, out);
+  };
+  switch (g) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 8: go(std::integral_constant<int, 8>{}); break;
+    case 16: go(std::integral_constant<int, 16>{}); break;
+    case 32: go(std::integral_constant<int, 32>{}); break;
+    default: go(std::integral_constant<int, 64>{}); break;
+  }
+  return true;
+}
+
 // The span route in one launch (one tile) or two (partials in `part`, folded and zeroed by the
 // second); `part_bytes` limits the tiles.
 template <class Op, class T>
@@ -1775,9 +1882,6 @@ void launch_reduce(const T* a, RedOut<T> out, int ndim, const size_t* shape, con
   // `tiles` is the caller's partial layout: every slot is written, tiles past the end of the
   // axis hold the operation's "empty" value
   constexpr int V = rvec<T>();
-  // reductions write next to nothing, so streaming loads win at every volume measured (the
-  // 128 MB c64 sum: 5.1 TB/s streaming vs 4.6 default), unlike the elementwise kernels
-  const bool nt = true;
   if constexpr (WRITE == kWriteFinal) {
     if (tiles == 1 && p.R > 0) {
       const ColRoute r = col_route(p, sizeof(T), Op::kOrdered);
@@ -1795,9 +1899,11 @@ void launch_reduce(const T* a, RedOut<T> out, int ndim, const size_t* shape, con
       }
     }
   }
+  if constexpr (WRITE == kWriteFinal && V > 1) {
+    if (tiles == 1 && launch_short<Op, T, V, T, T>(a, out, p, st)) return;
+  }
   if (p.kind == kColReduce && p.oshape[p.ond - 1] < (uint64_t(1) << 31)) {
     ColArgs ca{};
-    ca.nt = nt;
     ca.ix = out_indexer(p, p.ond - 1);
     ca.C = p.oshape[p.ond - 1];
     ca.cgroups = uint32_t(ceil_div(ca.C, uint64_t(kWave) * V));
@@ -1816,28 +1922,37 @@ void launch_reduce(const T* a, RedOut<T> out, int ndim, const size_t* shape, con
     return;
   }
   RowArgs ra{};
-  ra.nt = nt;
   ra.ix = out_indexer(p, p.ond);
   ra.R = p.R;
   ra.rs = p.rstride;
   ra.tiles = uint32_t(tiles);
   uint64_t chunk = ceil_div(p.R, tiles);
-  bool vec_ok = (p.rstride == 1) && al16(a);
+  const bool vec_ok = p.rstride == 1;  // rows may start at any element (vload_el)
+  bool aligned = al16(a);
   for (int d = 0; d < p.ond; ++d)
-    if ((uint64_t(p.ostride[d] < 0 ? -p.ostride[d] : p.ostride[d]) * sizeof(T)) % 16) vec_ok = false;
+    if ((uint64_t(p.ostride[d] < 0 ? -p.ostride[d] : p.ostride[d]) * sizeof(T)) % 16) aligned = false;
+  ra.nt = true;
   if (vec_ok && V > 1) chunk = ceil_div(chunk, V) * V;
   ra.chunk = chunk;
   ra.nwork = uint64_t(out_size) * tiles;
-  const uint64_t seg = chunk;
-  if (seg * sizeof(T) >= 16384) {  // >= 16 KB: a 512-lane block per segment
+  const uint64_t seg = chunk < p.R ? chunk : p.R;
+  // a 512-lane block per segment from 16 KB on; max / min / arg from 32 KB, since the few elements
+  // per lane of a shorter one improve the running extreme in nearly every chunk, and each time cost
+  // the search for its index ((16384, 4096) f32 max 65.2 us by blocks, 42.4 by waves; 32 KB rows of
+  // (8192, 8192) 40.1 by blocks, 43.8 by waves)
+  if (seg * sizeof(T) >= (Op::kOrdered ? 32768 : 16384)) {
     unsigned grid = unsigned(ra.nwork);
-    if (vec_ok)
+    if (vec_ok && aligned && chunk % (uint64_t(kRowBS) * V * 4) == 0 && p.R % chunk == 0)
+      k_reduce_row<Op, T, kRowBS, kRowBS, V, 4, WRITE, T, T, true><<<grid, kRowBS, 0, st>>>(a, ra, out);
+    else if (vec_ok)
       k_reduce_row<Op, T, kRowBS, kRowBS, V, 4, WRITE><<<grid, kRowBS, 0, st>>>(a, ra, out);
     else
       k_reduce_row<Op, T, kRowBS, kRowBS, 1, 8, WRITE><<<grid, kRowBS, 0, st>>>(a, ra, out);
   } else if (seg >= 64) {
     unsigned grid = unsigned(ceil_div(ra.nwork, kRBlock / kWave));
-    if (vec_ok)
+    if (vec_ok && Op::kOrdered && seg * sizeof(T) >= 16384)
+      k_reduce_row<Op, T, kRBlock, kWave, V, 4, WRITE><<<grid, kRBlock, 0, st>>>(a, ra, out);
+    else if (vec_ok)
       k_reduce_row<Op, T, kRBlock, kWave, V, 2, WRITE><<<grid, kRBlock, 0, st>>>(a, ra, out);
     else
       k_reduce_row<Op, T, kRBlock, kWave, 1, 4, WRITE><<<grid, kRBlock, 0, st>>>(a, ra, out);
@@ -1901,7 +2016,6 @@ int launch_reduce_col_last(const T* a, RedOut<T> out, const ReducePlan& p, size_
   if (p.oshape[p.ond - 1] >= (uint64_t(1) << 31) || ceil_div(p.R, uint64_t(tiles)) >= (uint64_t(1) << 31))
     return kFusedNotCovered;
   ColArgs ca{};
-  ca.nt = true;
   ca.ix = out_indexer(p, p.ond - 1);
   ca.C = p.oshape[p.ond - 1];
   ca.cgroups = uint32_t(ceil_div(ca.C, uint64_t(kWave) * V));
@@ -1951,9 +2065,7 @@ int launch_reduce_fused(const T* a, RedOut<T> out, int ndim, const size_t* shape
   if (out_size > kFusedMaxOutputs) return kFusedNotCovered;
   // 2048 tiles measured best for 64M f32 (a combiner lane then folds 4)
   if (tiles > kFusedMaxTiles) tiles = kFusedMaxTiles;
-  if (p.kind != kRowReduce || p.rstride != 1 || !al16(a)) return kFusedNotCovered;
-  for (int d = 0; d < p.ond; ++d)
-    if ((uint64_t(p.ostride[d] < 0 ? -p.ostride[d] : p.ostride[d]) * sizeof(T)) % 16) return kFusedNotCovered;
+  if (p.kind != kRowReduce || p.rstride != 1) return kFusedNotCovered;
   // one output over one contiguous run: the interleaved-chunk grid of launch_reduce_all_fused
   if (out_size == 1) {
     const int r = launch_reduce_all_fused<Op, OpF, T>(a, out, p.R, w, st);
@@ -1971,7 +2083,6 @@ int launch_reduce_fused(const T* a, RedOut<T> out, int ndim, const size_t* shape
   fa.fault = w.fault;
   fa.spin_limit = wait_spin_limit();
   RowArgs ra{};
-  ra.nt = true;
   ra.ix = out_indexer(p, p.ond);
   ra.R = p.R;
   ra.rs = 1;
@@ -2097,7 +2208,6 @@ int launch_reduce_2d_ordered(const T* a, RedOut<T> out, uint64_t R, uint64_t C, 
     }
   }
   ColArgs ca{};
-  ca.nt = true;
   ca.ix.nd = 0;
   ca.C = C;
   ca.cgroups = uint32_t(ceil_div(C, uint64_t(kWave) * V));

@@ -488,7 +488,7 @@ struct ColScanArgs {
 constexpr int kColWindow = 8;
 constexpr uint64_t kPrefixFlag = uint64_t(1) << 33;
 
-template <class T, int VE, int BS, int RPL, int LPC, bool CLAIM, bool NTS>
+template <class T, int VE, int BS, int RPL, int LPC, bool CLAIM, bool NTL, bool NTS>
 __global__ __launch_bounds__(BS) void k_scan_cols(const T* __restrict__ a, T* __restrict__ c, ColScanArgs sa) {
   using A = typename ScanAcc<T>::A;
   constexpr int SC = LPC * VE;              // columns of a tile
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(BS) void k_scan_cols(const T* __restrict__ a, T* __
 #pragma unroll
   for (int i = 0; i < RPL; ++i) {
     const uint64_t r = r0 + i < sa.L ? r0 + i : sa.L - 1;
-    d[i] = vload_el<T, VE>(ip + int64_t(r) * sa.ls_in, sa.nt_load);
+    d[i] = vload_el<T, VE, NTL>(ip + int64_t(r) * sa.ls_in);
   }
   A x[RPL][VE];
 #pragma unroll
@@ -871,16 +871,18 @@ void launch_scan_columns(const T* a, T* c, const ScanPlan& p, const ColScanRoute
   // Rows off 128-byte lines leave each run's end lines half written: default stores let the L2 of
   // the XCD that takes the neighbouring strip complete them.
   const bool lines = (uint64_t(sa.ls_out) * sizeof(T)) % 128 == 0 && (reinterpret_cast<uintptr_t>(c) & 127) == 0;
+  with_store_policy(sa.nt_load, [&](auto NTL) {
   with_store_policy(nts && lines, [&](auto NT) {
     if (sa.C < VE)
-      k_scan_cols<T, 1, kColBlockClaim, kColRpl, kColLpcThin, true, NT.value>
+      k_scan_cols<T, 1, kColBlockClaim, kColRpl, kColLpcThin, true, false, NT.value>
           <<<dim3(r.per * r.tiles), kColBlockClaim, 0, st>>>(a, c, sa);
     else if (r.claim)
-      k_scan_cols<T, VE, kColBlockClaim, kColRpl, kColLpc, true, NT.value>
+      k_scan_cols<T, VE, kColBlockClaim, kColRpl, kColLpc, true, NTL.value, NT.value>
           <<<dim3(r.per * r.tiles), kColBlockClaim, 0, st>>>(a, c, sa);
     else
-      k_scan_cols<T, VE, kColBlock, kColRpl, kColLpc, false, NT.value>
+      k_scan_cols<T, VE, kColBlock, kColRpl, kColLpc, false, NTL.value, NT.value>
           <<<dim3(r.per * r.tiles), kColBlock, 0, st>>>(a, c, sa);
+  });
   });
 }
 

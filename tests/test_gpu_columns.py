@@ -95,6 +95,39 @@ def test_column_results_repeat():
     assert_bits_equal(first[1], R.reduce(x, "argmax", 0), "argmax against the oracle")
 
 
+# ---- unit-stride rows that start and end anywhere ----
+@pytest.mark.parametrize("kind,dt", KINDS, ids=[f"{k}-{np.dtype(d).name}" for k, d in KINDS])
+def test_row_lengths(kind, dt):
+    """Every number of lanes per row with rows that end inside, at and after a vector (many short
+    rows), and the last round of the wave, block and tiled kernels."""
+    for shape in ((300001, 1), (140001, 3), (300003, 4), (140001, 5), (70001, 9), (70003, 16), (33001, 31),
+                  (17001, 67), (9001, 130), (9001, 257), (4500, 513), (300, 1013), (70, 4097), (40, 8195),
+                  (16, 16384), (3, 70001), (5, 40003)):
+        if dt not in (np.float32, np.int64) and shape[0] > 20000:
+            continue
+        check_reduce(kind, values(kind, dt, shape), 1)
+
+
+@pytest.mark.parametrize("kind", ["sum", "max", "argmin"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_row_views_and_ordered_semantics(kind, dt):
+    base = RNG.integers(-2, 3, (9001, 261)).astype(dt)
+    if kind != "sum":
+        base[::5, 0] = np.nan
+        base[1::3, 100] = np.nan
+        base[2::7, 1:] = np.nan
+        base[3::7, -1] = -0.0
+    B = dev(base)
+    check_reduce(kind, base, 1)
+    for lo, hi, step in ((1, 36, 1), (0, 133, 1), (3, 260, 1), (2, 258, 1), (0, 261, 3)):
+        check_reduce(kind, np.ascontiguousarray(base[:, lo:hi:step]), 1,
+                     gpu_x=ms.slice(B, [(0, 9001, 1), (lo, hi, step)]))
+    long = RNG.integers(-2, 3, (5, 70003)).astype(dt)
+    if kind != "sum":
+        long[0, 0], long[1, -1] = np.nan, np.nan
+    check_reduce(kind, np.ascontiguousarray(long[:, 1:]), 1, gpu_x=ms.slice(dev(long), [(0, 5, 1), (1, 70003, 1)]))
+
+
 # ---- cumsum down the columns ----
 SCAN_SHAPES = [
     ((63, 5), 0), ((64, 3), 0), ((384, 70), 0),                    # sequential, one lane per column
