@@ -63,13 +63,13 @@ __global__ __launch_bounds__(kFlatBlockUnary) void k_unary_flat(In<TA> a, TO* __
         for (int k = 0; k < VEC; ++k) va[u].v[k] = s;
     } else {
       static_for<UNROLL>(
-          [&](auto u) { va[u] = vload_pol<TA, VEC>(a.p + base + uint64_t(u * kFlatBlockUnary + t) * VEC, a.nt); });
+          [&](auto u) { va[u] = vload_el_pol<TA, VEC>(a.p + base + uint64_t(u * kFlatBlockUnary + t) * VEC, a.nt); });
     }
     static_for<UNROLL>([&](auto u) {
       Vec<TO, VEC> vc;
 #pragma unroll
       for (int k = 0; k < VEC; ++k) vc.v[k] = f(va[u].v[k]);
-      vstore_as<NTS, TO, VEC>(c + base + uint64_t(u * kFlatBlockUnary + t) * VEC, vc);
+      vstore_el<NTS, TO, VEC>(c + base + uint64_t(u * kFlatBlockUnary + t) * VEC, vc);
     });
   } else {
     for (uint64_t i = base + t; i < n; i += kFlatBlockUnary) c[i] = f(a.mode == kModeScalar ? a.p[0] : a.p[i]);
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(kFlatBlockBinary) void k_binary_flat(In<T> a, In<T>
         for (int k = 0; k < VEC; ++k) va[u].v[k] = s;
     } else {
       static_for<UNROLL>(
-          [&](auto u) { va[u] = vload_pol<T, VEC>(a.p + base + uint64_t(u * kFlatBlockBinary + t) * VEC, a.nt); });
+          [&](auto u) { va[u] = vload_el_pol<T, VEC>(a.p + base + uint64_t(u * kFlatBlockBinary + t) * VEC, a.nt); });
     }
     if (b.mode == kModeScalar) {
       const T s = b.p[0];
@@ -103,13 +103,13 @@ __global__ __launch_bounds__(kFlatBlockBinary) void k_binary_flat(In<T> a, In<T>
         for (int k = 0; k < VEC; ++k) vb[u].v[k] = s;
     } else {
       static_for<UNROLL>(
-          [&](auto u) { vb[u] = vload_pol<T, VEC>(b.p + base + uint64_t(u * kFlatBlockBinary + t) * VEC, b.nt); });
+          [&](auto u) { vb[u] = vload_el_pol<T, VEC>(b.p + base + uint64_t(u * kFlatBlockBinary + t) * VEC, b.nt); });
     }
     static_for<UNROLL>([&](auto u) {
       Vec<TO, VEC> vc;
 #pragma unroll
       for (int k = 0; k < VEC; ++k) vc.v[k] = f(va[u].v[k], vb[u].v[k]);
-      vstore_as<NTS, TO, VEC>(c + base + uint64_t(u * kFlatBlockBinary + t) * VEC, vc);
+      vstore_el<NTS, TO, VEC>(c + base + uint64_t(u * kFlatBlockBinary + t) * VEC, vc);
     });
   } else {
     for (uint64_t i = base + t; i < n; i += kFlatBlockBinary)
@@ -119,9 +119,12 @@ __global__ __launch_bounds__(kFlatBlockBinary) void k_binary_flat(In<T> a, In<T>
 
 // ---------------------------------------------------------------------------------------------
 // rows: output rows of length L (the innermost coalesced dim).  A work item is VEC consecutive
-// elements of one row; `aligned` (host-checked) guarantees every item is full and every
-// unit-stride operand is 16-byte aligned at the item start.
-// nt: streaming loads; false for operands that every block re-reads (broadcast rows).
+// elements of one row, loaded and stored as element-aligned vectors (rows of odd length, slices
+// that start anywhere); only the last, partial item of a row (`full` false) goes element by element.
+// HBM-bound.  When rows off 16 bytes went element by element instead, four loads and stores per lane
+// of which each touched every line of the wave's run, x - row of (20011, 3001) f32 took 191 us and now
+// takes 84 (5.7 TB/s), neighbours along rows of 4003 f32 103 and now 50, f64 119 and 91, and abs of
+// (4097, 7999) f32 slices 80 and 44.
 template <int VEC, class T>
 __device__ inline void load_item(const T* base, int mode, int64_t s, uint32_t col, uint32_t L, bool full, bool nt,
                                  T (&x)[VEC]) {
@@ -130,12 +133,12 @@ __device__ inline void load_item(const T* base, int mode, int64_t s, uint32_t co
 #pragma unroll
     for (int k = 0; k < VEC; ++k) x[k] = v;
   } else if (mode == kModeUnit && full) {
-    Vec<T, VEC> v = vload_pol<T, VEC>(base + col, nt);
+    Vec<T, VEC> v = vload_el_pol<T, VEC>(base + col, nt);
 #pragma unroll
     for (int k = 0; k < VEC; ++k) x[k] = v.v[k];
   } else if (mode == kModeRev && full) {
     // elements col .. col+VEC-1 of the row sit at base-col-(VEC-1) .. base-col
-    Vec<T, VEC> v = vload_pol<T, VEC>(base - (int64_t(col) + (VEC - 1)), nt);
+    Vec<T, VEC> v = vload_el_pol<T, VEC>(base - (int64_t(col) + (VEC - 1)), nt);
 #pragma unroll
     for (int k = 0; k < VEC; ++k) x[k] = v.v[VEC - 1 - k];
   } else {
@@ -152,7 +155,7 @@ constexpr int kRowsBlock = 128;
 constexpr int kRowsUnroll = 4;
 template <int VEC, int UNROLL, bool NTS, class F, class TO, class TA>
 __global__ __launch_bounds__(kRowsBlock) void k_unary_rows(In<TA> a, int64_t sa, TO* __restrict__ c, RowIndexer<2> ix,
-                                                           FastDiv gpr, uint32_t L, uint32_t items, bool aligned, F f) {
+                                                           FastDiv gpr, uint32_t L, uint32_t items, F f) {
   const uint32_t first = blockIdx.x * (kRowsBlock * UNROLL) + threadIdx.x;
 #pragma unroll
   for (int u = 0; u < UNROLL; ++u) {
@@ -162,15 +165,15 @@ __global__ __launch_bounds__(kRowsBlock) void k_unary_rows(In<TA> a, int64_t sa,
     const uint32_t col = (g - row * gpr.d) * VEC;
     int64_t off[2];
     row_offsets<2>(ix, row, off);
-    const bool full = aligned || (col + VEC <= L);
+    const bool full = col + VEC <= L;
     TA x[VEC];
-    load_item<VEC, TA>(a.p + off[1], a.mode, sa, col, L, full && aligned, a.nt, x);
+    load_item<VEC, TA>(a.p + off[1], a.mode, sa, col, L, full, a.nt, x);
     TO* cp = c + off[0] + col;
-    if (full && aligned) {
+    if (full) {
       Vec<TO, VEC> v;
 #pragma unroll
       for (int k = 0; k < VEC; ++k) v.v[k] = f(x[k]);
-      vstore_as<NTS, TO, VEC>(cp, v);
+      vstore_el<NTS, TO, VEC>(cp, v);
     } else {
 #pragma unroll
       for (int k = 0; k < VEC; ++k)
@@ -182,7 +185,7 @@ __global__ __launch_bounds__(kRowsBlock) void k_unary_rows(In<TA> a, int64_t sa,
 template <int VEC, int UNROLL, bool NTS, class F, class T, class TO = T>
 __global__ __launch_bounds__(kBlock) void k_binary_rows(In<T> a, int64_t sa, In<T> b, int64_t sb, TO* __restrict__ c,
                                                         RowIndexer<3> ix, FastDiv gpr, uint32_t L, uint32_t items,
-                                                        bool aligned, F f) {
+                                                        F f) {
   const uint32_t first = blockIdx.x * (kBlock * UNROLL) + threadIdx.x;
 #pragma unroll
   for (int u = 0; u < UNROLL; ++u) {
@@ -192,16 +195,16 @@ __global__ __launch_bounds__(kBlock) void k_binary_rows(In<T> a, int64_t sa, In<
     const uint32_t col = (g - row * gpr.d) * VEC;
     int64_t off[3];
     row_offsets<3>(ix, row, off);
-    const bool full = aligned || (col + VEC <= L);
+    const bool full = col + VEC <= L;
     T x[VEC], y[VEC];
-    load_item<VEC, T>(a.p + off[1], a.mode, sa, col, L, full && aligned, a.nt, x);
-    load_item<VEC, T>(b.p + off[2], b.mode, sb, col, L, full && aligned, b.nt, y);
+    load_item<VEC, T>(a.p + off[1], a.mode, sa, col, L, full, a.nt, x);
+    load_item<VEC, T>(b.p + off[2], b.mode, sb, col, L, full, b.nt, y);
     TO* cp = c + off[0] + col;
-    if (full && aligned) {
+    if (full) {
       Vec<TO, VEC> v;
 #pragma unroll
       for (int k = 0; k < VEC; ++k) v.v[k] = f(x[k], y[k]);
-      vstore_as<NTS, TO, VEC>(cp, v);
+      vstore_el<NTS, TO, VEC>(cp, v);
     } else {
 #pragma unroll
       for (int k = 0; k < VEC; ++k)
@@ -221,12 +224,12 @@ __global__ __launch_bounds__(kFlatBlockMixed) void k_binary_flat_mixed(const TA*
   const CastF<TA, TC> ca{};
   const CastF<TB, TC> cb{};
   if (i0 + VEC <= n) {
-    Vec<TA, VEC> x = vload_pol<TA, VEC>(a + i0, nt);
-    Vec<TB, VEC> y = vload_pol<TB, VEC>(b + i0, nt);
+    Vec<TA, VEC> x = vload_el_pol<TA, VEC>(a + i0, nt);
+    Vec<TB, VEC> y = vload_el_pol<TB, VEC>(b + i0, nt);
     Vec<TC, VEC> z;
 #pragma unroll
     for (int k = 0; k < VEC; ++k) z.v[k] = f(ca(x.v[k]), cb(y.v[k]));
-    vstore_as<NTS, TC, VEC>(c + i0, z);
+    vstore_el<NTS, TC, VEC>(c + i0, z);
   } else {
     for (uint64_t i = i0; i < n; ++i) c[i] = f(ca(a[i]), cb(b[i]));
   }
@@ -248,7 +251,6 @@ struct RowPieceArgs {
   RowIndexer<3> ix;   // outer dims: [0] out, [1] a, [2] b strides
   uint32_t L;         // row length (innermost output dim)
   FastDiv groups;     // blocks per row
-  bool aligned;       // every item full and 16-byte aligned (host-checked)
 };
 
 template <int VEC, int U, bool NTS, class F, class T, class TO = T>
@@ -263,20 +265,20 @@ __global__ __launch_bounds__(kPieceBlock) void k_binary_rowpieces(In<T> a, int64
   for (int u = 0; u < U; ++u) {
     const uint32_t col = ((g * U + u) * kPieceBlock + threadIdx.x) * VEC;
     if (col >= ra.L) break;
-    const bool full = ra.aligned || col + VEC <= ra.L;
-    load_item<VEC, T>(a.p + off[1], a.mode, sa, col, ra.L, full && ra.aligned, a.nt, xa[u]);
-    load_item<VEC, T>(b.p + off[2], b.mode, sb, col, ra.L, full && ra.aligned, b.nt, xb[u]);
+    const bool full = col + VEC <= ra.L;
+    load_item<VEC, T>(a.p + off[1], a.mode, sa, col, ra.L, full, a.nt, xa[u]);
+    load_item<VEC, T>(b.p + off[2], b.mode, sb, col, ra.L, full, b.nt, xb[u]);
   }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const uint32_t col = ((g * U + u) * kPieceBlock + threadIdx.x) * VEC;
     if (col >= ra.L) break;
     TO* cp = c + off[0] + col;
-    if (ra.aligned) {
+    if (col + VEC <= ra.L) {
       Vec<TO, VEC> v;
 #pragma unroll
       for (int k = 0; k < VEC; ++k) v.v[k] = f(xa[u][k], xb[u][k]);
-      vstore_as<NTS, TO, VEC>(cp, v);
+      vstore_el<NTS, TO, VEC>(cp, v);
     } else {
 #pragma unroll
       for (int k = 0; k < VEC; ++k)
@@ -294,7 +296,6 @@ struct TransposeArgs {
   int64_t out_sP;          // output stride along P (output stride along L is 1)
   FastDiv tilesL, tilesP;  // tile counts
   RowIndexer<2> batch;     // batch dims: [0] output strides, [1] input strides
-  bool vec_in, vec_out;    // 16-byte aligned vector access possible on each side
   bool nt;                 // streaming loads
   bool pmajor;             // consecutive blocks take consecutive tiles along P (else along L)
 };
@@ -374,30 +375,38 @@ __global__ __launch_bounds__(BS) void k_unary_transpose(const TI* __restrict__ a
     const int pp = (t % PL) * VI;
     const int lr = t / PL;
     const uint64_t p = p0 + pp;
-    if (ta.vec_in && l0 + TL <= ta.L && p0 + TP <= ta.P) {
+    if (l0 + TL <= ta.L && p0 + TP <= ta.P) {
       // interior tile: every pass's load is issued before the first LDS store
       Vec<TI, VI> v[NRP];
 #pragma unroll
       for (int k = 0; k < NRP; ++k)
-        v[k] = vload_pol<TI, VI>(ab + int64_t(l0 + lr + k * RP) * ta.in_sL + int64_t(p), ta.nt);
+        v[k] = vload_el_pol<TI, VI>(ab + int64_t(l0 + lr + k * RP) * ta.in_sL + int64_t(p), ta.nt);
 #pragma unroll
       for (int k = 0; k < NRP; ++k)
 #pragma unroll
         for (int q = 0; q < VI; ++q) tile[lr + k * RP][pp + q] = f(v[k].v[q]);
     } else {
-      for (int ll = lr; ll < TL; ll += RP) {
-        const uint64_t l = l0 + ll;
-        if (l >= ta.L) break;
-        const TI* src = ab + int64_t(l) * ta.in_sL + int64_t(p);
-        if (ta.vec_in && p + VI <= ta.P) {
-          Vec<TI, VI> v = vload_pol<TI, VI>(src, ta.nt);
+      // edge tile: likewise, up to the array's ends
+      Vec<TI, VI> v[NRP];
 #pragma unroll
-          for (int q = 0; q < VI; ++q) tile[ll][pp + q] = f(v.v[q]);
+      for (int k = 0; k < NRP; ++k) {
+        const uint64_t l = l0 + lr + k * RP;
+        if (l >= ta.L) continue;
+        const TI* src = ab + int64_t(l) * ta.in_sL + int64_t(p);
+        if (p + VI <= ta.P) {
+          v[k] = vload_el_pol<TI, VI>(src, ta.nt);
         } else {
 #pragma unroll
           for (int q = 0; q < VI; ++q)
-            if (p + q < ta.P) tile[ll][pp + q] = f(src[q]);
+            if (p + q < ta.P) v[k].v[q] = src[q];
         }
+      }
+#pragma unroll
+      for (int k = 0; k < NRP; ++k) {
+        if (l0 + lr + k * RP >= ta.L) break;
+#pragma unroll
+        for (int q = 0; q < VI; ++q)
+          if (p + q < ta.P) tile[lr + k * RP][pp + q] = f(v[k].v[q]);
       }
     }
   }
@@ -410,11 +419,11 @@ __global__ __launch_bounds__(BS) void k_unary_transpose(const TI* __restrict__ a
       const uint64_t p = p0 + pp;
       if (p >= ta.P) break;
       TO* dst = cb + int64_t(p) * ta.out_sP + int64_t(l);
-      if (ta.vec_out && l + VO <= ta.L) {
+      if (l + VO <= ta.L) {
         Vec<TO, VO> v;
 #pragma unroll
         for (int q = 0; q < VO; ++q) v.v[q] = tile[ll + q][pp];
-        vstore_as<NTS, TO, VO>(dst, v);
+        vstore_el<NTS, TO, VO>(dst, v);
       } else {
 #pragma unroll
         for (int q = 0; q < VO; ++q)
@@ -546,8 +555,6 @@ constexpr int ew_vec() {
   return (sizeof(TA) <= 2 && sizeof(TA) * vo < 8) ? 2 * vo : vo;
 }
 
-inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
 inline int mode_of(int64_t s) {
   return s == 0 ? kModeScalar : (s == 1 ? kModeUnit : (s == -1 ? kModeRev : kModeStrided));
 }
@@ -570,6 +577,34 @@ inline uint64_t operand_elems(const Plan& p, int o) {
   return n;
 }
 
+// true when every row that operand `o` walks starts on a 128-byte line.  Only then do streaming loads
+// pay: a row that starts inside a line shares its first and last line with its neighbours, and a
+// streamed line is not kept for them.  Measured with rotated buffers, default against streaming
+// loads: x - row of (20011, 3001) 87.6 against 95.1 us in f32 and 210 against 225 in f64, (20000,
+// 3000) f64 196 against 215, neighbours along rows of 4003 f64 90 against 106, but the sum with a
+// transposed (8192, 4096) operand 75.4 against 71.1 us in f32 and 144 against 135 in f64, and exp
+// of that view 102 against 97 us in f64.
+template <class T>
+inline bool at_lines(const Plan& p, int o, const void* ptr) {
+  const int64_t es = int64_t(sizeof(T));
+  uintptr_t q = reinterpret_cast<uintptr_t>(ptr);
+  for (int d = 0; d < p.ndim; ++d) {
+    const int64_t s = p.stride[o][d];
+    if (s == -1) q -= (p.shape[d] - 1) * sizeof(T);  // a flipped row starts at its far end
+    if (s < -1 || s > 1)
+      if (s * es % 128) return false;
+  }
+  return q % 128 == 0;
+}
+
+// Output rows off 16 bytes are streamed beside a large input only: next to it streaming measured
+// up to 20% faster (abs of (4097, 7999) slices 54.9 -> 43.7 us), but a lone output, whose lines at
+// the row ends then go out in parts, slower (the outer difference of 8009 and 4003 f64 49.0 -> 59.8).
+template <class TO>
+inline bool out_aligned(const Plan& p, const void* c) {
+  return p.shape[p.ndim - 1] * sizeof(TO) % 16 == 0 && reinterpret_cast<uintptr_t>(c) % 16 == 0;
+}
+
 inline unsigned grid_generic(uint64_t n) {
   uint64_t g = (n + kBlock - 1) / kBlock;
   return unsigned(g > 65536 ? 65536 : g);
@@ -586,28 +621,6 @@ inline bool rows_ok(const Plan& p, int vec) {
   return true;
 }
 
-// true when every unit-stride (or reversed, stride -1) operand has each VEC item of every row
-// on one aligned vector: 16 bytes, or the item's size when that is smaller
-template <class T0, class T1, class T2 = T1>
-inline bool rows_aligned(const Plan& p, int vec, const void* c, const void* a, const void* b = nullptr) {
-  uint64_t L = p.shape[p.ndim - 1];
-  if (L % vec) return false;
-  const void* ptr[3] = {c, a, b};
-  const size_t es[3] = {sizeof(T0), sizeof(T1), sizeof(T2)};
-  for (int o = 0; o < p.nops; ++o) {
-    int64_t s = p.stride[o][p.ndim - 1];
-    if (s != 1 && s != -1) continue;
-    // a reversed row's first item ends at the row start: its vector starts vec-1 elements lower
-    const uintptr_t q = reinterpret_cast<uintptr_t>(ptr[o]) - (s == -1 ? (vec - 1) * es[o] : 0);
-    if (es[o] * vec < 16 ? (q % (es[o] * vec)) : (q % 16)) return false;
-    for (int d = 0; d < p.ndim - 1; ++d) {
-      uint64_t bytes = uint64_t(p.stride[o][d] < 0 ? -p.stride[o][d] : p.stride[o][d]) * es[o];
-      if (bytes % (es[o] * vec < 16 ? es[o] * vec : 16)) return false;
-    }
-  }
-  return true;
-}
-
 template <class F, class TO, class TA>
 void launch_unary(const TA* a, TO* c, int ndim, const size_t* shape, const ssize_t* as, hipStream_t st, F f) {
   Plan p;
@@ -615,22 +628,17 @@ void launch_unary(const TA* a, TO* c, int ndim, const size_t* shape, const ssize
   if (!args_ok(ndim) || !plan_elementwise(p, ndim, shape, 1, ins)) return;
   // the narrower type moves 16 bytes per item, the wider one 16-32 (e.g. f64->f32: 4 elements)
   constexpr int V = ew_vec<TA, TO>();
-  const bool nt = operand_elems(p, 1) * sizeof(TA) >= kStreamLoadBytes;
-  const bool nts = p.numel * sizeof(TO) >= kStreamStoreBytesUnary;
+  const bool big = operand_elems(p, 1) * sizeof(TA) >= kStreamLoadBytes;
+  const bool nt = big && at_lines<TA>(p, 1, a);
+  const bool nts = p.numel * sizeof(TO) >= kStreamStoreBytesUnary && (big || out_aligned<TO>(p, c));
   if (p.ndim == 1 && p.stride[0][0] == 1 && (p.stride[1][0] == 0 || p.stride[1][0] == 1)) {
     In<TA> ia{a, mode_of(p.stride[1][0]), nt};
-    bool vec_ok = aligned16(c) && (ia.mode == kModeScalar || aligned16(a));
-    if (vec_ok) {
-      constexpr uint64_t kTile = uint64_t(kFlatBlockUnary) * V * kFlatUnroll;
-      const uint64_t tiles = (p.numel + kTile - 1) / kTile;
-      with_store_policy(nts, [&](auto NT) {
-        k_unary_flat<V, kFlatUnroll, NT.value, F, TO, TA><<<dim3(unsigned(tiles)), kFlatBlockUnary, 0, st>>>(
-            ia, c, p.numel, f);
-      });
-    } else {
-      uint64_t tiles = (p.numel + uint64_t(kFlatBlockUnary) * kUnroll - 1) / (uint64_t(kFlatBlockUnary) * kUnroll);
-      k_unary_flat<1, kUnroll, false, F, TO, TA><<<dim3(unsigned(tiles)), kFlatBlockUnary, 0, st>>>(ia, c, p.numel, f);
-    }
+    constexpr uint64_t kTile = uint64_t(kFlatBlockUnary) * V * kFlatUnroll;
+    const uint64_t tiles = (p.numel + kTile - 1) / kTile;
+    with_store_policy(nts, [&](auto NT) {
+      k_unary_flat<V, kFlatUnroll, NT.value, F, TO, TA><<<dim3(unsigned(tiles)), kFlatBlockUnary, 0, st>>>(
+          ia, c, p.numel, f);
+    });
     return;
   }
   // transposed input: unit stride along some dim other than the innermost one
@@ -650,19 +658,16 @@ void launch_unary(const TA* a, TO* c, int ndim, const size_t* shape, const ssize
       {
         // batch dims: all dims but P and nd-1, innermost first
         ta.batch.nd = 0;
-        ta.vec_in = aligned16(a) && (uint64_t(sL < 0 ? -sL : sL) * sizeof(TA)) % 16 == 0;
-        ta.vec_out = aligned16(c) && (uint64_t(ta.out_sP) * sizeof(TO)) % 16 == 0;
         // tiles read across many rows at once: streaming won at 128 MB too (5.1 vs 4.9 TB/s), and with
-        // the 1024-lane tiles default loads ran 2-8% slower (f32 X^T 98.1 vs 91.2 us, c128 98.9 vs 91.4)
-        ta.nt = true;
+        // the 1024-lane tiles default loads ran 2-8% slower (f32 X^T 98.1 vs 91.2 us, c128 98.9 vs 91.4);
+        // rows off the lines take default loads at any size, see at_lines()
+        ta.nt = at_lines<TA>(p, 1, a);
         for (int d = nd - 2; d >= 0; --d) {
           if (d == P) continue;
           int k = ta.batch.nd++;
           ta.batch.div[k] = make_fastdiv(uint32_t(p.shape[d]));
           ta.batch.stride[0][k] = p.stride[0][d];
           ta.batch.stride[1][k] = p.stride[1][d];
-          if ((uint64_t(p.stride[1][d] < 0 ? -p.stride[1][d] : p.stride[1][d]) * sizeof(TA)) % 16) ta.vec_in = false;
-          if ((uint64_t(p.stride[0][d]) * sizeof(TO)) % 16) ta.vec_out = false;
         }
         if (launch_transpose<F, TO, TA>(a, c, ta, nb, nts, st, f)) return;
       }
@@ -671,14 +676,13 @@ void launch_unary(const TA* a, TO* c, int ndim, const size_t* shape, const ssize
   if ((nd >= 2 || sL == -1) && rows_ok(p, V)) {
     const uint32_t L = uint32_t(p.shape[nd - 1]);
     In<TA> ia{a, mode_of(sL), nt};
-    bool al = rows_aligned<TO, TA>(p, V, c, a);
     uint32_t gpr = (L + V - 1) / V;
     uint32_t items = uint32_t(p.numel / L) * gpr;
     RowIndexer<2> ix = make_row_indexer<2>(p);
     unsigned grid = (items + kRowsBlock * kRowsUnroll - 1) / (kRowsBlock * kRowsUnroll);
     with_store_policy(nts, [&](auto NT) {
       k_unary_rows<V, kRowsUnroll, NT.value, F, TO, TA><<<grid, kRowsBlock, 0, st>>>(ia, sL, c, ix, make_fastdiv(gpr),
-                                                                                   L, items, al, f);
+                                                                                   L, items, f);
     });
     return;
   }
@@ -693,32 +697,23 @@ void launch_binary(const T* a, const T* b, TO* c, int ndim, const size_t* shape,
   if (!args_ok(ndim) || !plan_elementwise(p, ndim, shape, 2, ins)) return;
   constexpr int V = vec_of<T>();
   const int nd = p.ndim;
-  const bool nt = (operand_elems(p, 1) + operand_elems(p, 2)) * sizeof(T) >= kStreamLoadBytes;
-  const bool nts = p.numel * sizeof(TO) >= kStreamStoreBytes;
+  const bool big = (operand_elems(p, 1) + operand_elems(p, 2)) * sizeof(T) >= kStreamLoadBytes;
+  const bool nt = big && at_lines<T>(p, 1, a) && at_lines<T>(p, 2, b);
+  const bool nts = p.numel * sizeof(TO) >= kStreamStoreBytes && (big || out_aligned<TO>(p, c));
   if (nd == 1 && (p.stride[1][0] == 0 || p.stride[1][0] == 1) && (p.stride[2][0] == 0 || p.stride[2][0] == 1)) {
     In<T> ia{a, mode_of(p.stride[1][0]), nt}, ib{b, mode_of(p.stride[2][0]), nt};
-    constexpr uintptr_t kOutAlign = sizeof(TO) * V < 16 ? sizeof(TO) * V : 16;  // one output vector
-    bool vec_ok = (reinterpret_cast<uintptr_t>(c) % kOutAlign) == 0 && (ia.mode == kModeScalar || aligned16(a)) &&
-                  (ib.mode == kModeScalar || aligned16(b));
-    if (vec_ok) {
-      constexpr uint64_t kTile = uint64_t(kFlatBlockBinary) * V * kFlatUnroll;
-      const uint64_t tiles = (p.numel + kTile - 1) / kTile;
-      with_store_policy(nts, [&](auto NT) {
-        k_binary_flat<V, kFlatUnroll, NT.value, F, T, TO><<<dim3(unsigned(tiles)), kFlatBlockBinary, 0, st>>>(
-            ia, ib, c, p.numel, f);
-      });
-    } else {
-      uint64_t tiles = (p.numel + uint64_t(kFlatBlockBinary) * kUnroll - 1) / (uint64_t(kFlatBlockBinary) * kUnroll);
-      k_binary_flat<1, kUnroll, false, F, T, TO><<<dim3(unsigned(tiles)), kFlatBlockBinary, 0, st>>>(ia, ib, c,
-                                                                                                     p.numel, f);
-    }
+    constexpr uint64_t kTile = uint64_t(kFlatBlockBinary) * V * kFlatUnroll;
+    const uint64_t tiles = (p.numel + kTile - 1) / kTile;
+    with_store_policy(nts, [&](auto NT) {
+      k_binary_flat<V, kFlatUnroll, NT.value, F, T, TO><<<dim3(unsigned(tiles)), kFlatBlockBinary, 0, st>>>(
+          ia, ib, c, p.numel, f);
+    });
     return;
   }
   if (rows_ok(p, V)) {
     const uint32_t L = uint32_t(p.shape[nd - 1]);
     const int64_t sa = p.stride[1][nd - 1], sb = p.stride[2][nd - 1];
     In<T> ia{a, mode_of(sa), nt}, ib{b, mode_of(sb), nt};
-    bool al = rows_aligned<TO, T, T>(p, V, c, a, b);
     uint32_t gpr = (L + V - 1) / V;
     uint32_t items = uint32_t(p.numel / L) * gpr;
     RowIndexer<3> ix = make_row_indexer<3>(p);
@@ -728,7 +723,6 @@ void launch_binary(const T* a, const T* b, TO* c, int ndim, const size_t* shape,
       RowPieceArgs ra{};
       ra.ix = ix;
       ra.L = L;
-      ra.aligned = al;
       const uint32_t groups = (L + uint32_t(kPieceBlock) * V * U - 1) / (uint32_t(kPieceBlock) * V * U);
       ra.groups = make_fastdiv(groups);
       const uint64_t blocks = uint64_t(p.numel / L) * groups;
@@ -743,7 +737,7 @@ void launch_binary(const T* a, const T* b, TO* c, int ndim, const size_t* shape,
     unsigned grid = (items + kBlock * kUnroll - 1) / (kBlock * kUnroll);
     with_store_policy(nts, [&](auto NT) {
       k_binary_rows<V, kUnroll, NT.value, F, T, TO><<<grid, kBlock, 0, st>>>(ia, sa, ib, sb, c, ix, make_fastdiv(gpr),
-                                                                           L, items, al, f);
+                                                                           L, items, f);
     });
     return;
   }
@@ -761,9 +755,10 @@ void launch_binary_mixed(const void* a, const void* b, void* c, int ndim, const 
   TC* pc = static_cast<TC*>(c);
   constexpr int V = 16 / (sizeof(TA) > sizeof(TB) ? (sizeof(TA) > sizeof(TC) ? sizeof(TA) : sizeof(TC))
                                                   : (sizeof(TB) > sizeof(TC) ? sizeof(TB) : sizeof(TC)));
-  if (p.ndim == 1 && p.stride[1][0] == 1 && p.stride[2][0] == 1 && aligned16(a) && aligned16(b) && aligned16(c)) {
+  if (p.ndim == 1 && p.stride[1][0] == 1 && p.stride[2][0] == 1) {
     const uint64_t blocks = (p.numel + uint64_t(kFlatBlockMixed) * V - 1) / (uint64_t(kFlatBlockMixed) * V);
-    const bool nt = p.numel * (sizeof(TA) + sizeof(TB)) >= kStreamLoadBytes;
+    const bool nt = p.numel * (sizeof(TA) + sizeof(TB)) >= kStreamLoadBytes && at_lines<TA>(p, 1, a) &&
+                    at_lines<TB>(p, 2, b);
     const bool nts = p.numel * sizeof(TC) >= kStreamStoreBytes;
     with_store_policy(nts, [&](auto NT) {
       k_binary_flat_mixed<V, NT.value, F, TC, TA, TB><<<dim3(unsigned(blocks)), kFlatBlockMixed, 0, st>>>(

@@ -170,6 +170,18 @@ __device__ inline void vstore_el(T* p, const Vec<T, N>& v) {
   }
 }
 
+// By a runtime flag: the default load copies elements where the streaming one loads words, so that
+// the compiler keeps both (tests/test_streaming_stores.py looks at the build).
+template <typename T, int N>
+__device__ inline Vec<T, N> vload_el_pol(const T* p, bool nt) {
+  struct El { T v[N]; };
+  if (nt) return vload_el<T, N, true>(p);
+  const El e = *reinterpret_cast<const El*>(p);
+  Vec<T, N> v;
+#pragma unroll
+  for (int k = 0; k < N; ++k) v.v[k] = e.v[k];
+  return v;
+}
 template <typename T, int N>
 __device__ inline Vec<T, N> vload_pol(const T* p, bool nt) {
   return nt ? vload_nt<T, N>(p) : vload<T, N>(p);
