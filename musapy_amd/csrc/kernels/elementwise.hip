@@ -8,6 +8,7 @@
 //              per lane, many short blocks;
 //   tiles      (binary, long rows) column tiles that walk down the rows: an operand broadcast
 //              along the rows stays in registers, a per-row scalar costs one load per row;
+//   binary transpose  binary ops of one such view and an operand laid out like the output;
 //   rows       output rows of the innermost dim; the outer coordinates of a row are decoded
 //              once with 32-bit magic division, the inner dim is streamed per operand as
 //              vector (stride 1), broadcast (stride 0) or gather (any other stride);
@@ -481,6 +482,203 @@ bool launch_transpose(const TI* a, TO* c, TransposeArgs ta, uint64_t nb, bool nt
 }
 
 // ---------------------------------------------------------------------------------------------
+// binary ops of a transposed operand x (unit stride along a dim P that is not the innermost dim L)
+// and one that is unit-stride or constant along L (y): the tile of x goes through LDS as above, y's
+// vectors are loaded in the output's layout before the barrier, so both streams are in flight
+// together, and the functor runs on the store side.  HBM-bound; the row kernels, which gather x one
+// element per row of it, read every line of x from L2 once per element.  Sum of a (6000, 5000) array
+// and a transposed view, with rotated buffers: 291 -> 78 us in f32 (4.6 TB/s), 444 -> 136 in f64;
+// (8192, 4096) 282 -> 71 and 278 -> 135; (300, 60000) f32 246 -> 44; (1000, 700) f32 9.4 -> 4.2.
+// Consecutive blocks take consecutive tiles along L, which two of the three streams follow (along P:
+// 83.5 against 78.1 us at (6000, 5000) f32, 87 against 75 at (8192, 4096)).  Tiles:
+//  * 32 lanes x 128 rows, 1024 lanes: large arrays (the small tile 88 us at (6000, 5000) f32);
+//  * 8 lanes x 64 rows, 256 lanes: below 4M elements, where the large tile leaves CUs idle ((1000,
+//    700) 4.2 against 6.1 us), and dims of up to 64, half of the large tile ((200000, 37) f32 19.3
+//    against 25.5 us, (16, 200000) 8.4 against 16.3);
+//  * 64 lanes x 32 rows, 512 lanes: L of up to 32 ((200000, 16) f32 10.5 us, small tile 11.2, large
+//    17.6).
+// P and L below 16 keep the row kernels: such tiles would be mostly empty.
+constexpr uint64_t kBinTransposeMin = 16;
+constexpr uint64_t kBinTransposeSmall = uint64_t(4) << 20;
+struct BinTransposeArgs {
+  uint64_t P, L;
+  int64_t x_sL;            // stride of x along L (1 along P)
+  int64_t y_sP;            // stride of y along P
+  bool y_unit;             // y has unit stride along L; otherwise it is constant along L
+  int64_t out_sP;
+  FastDiv tilesL, tilesP;
+  RowIndexer<3> batch;     // batch dims: [0] out, [1] x, [2] y strides
+  bool swap;               // x is the second operand
+  bool nt;                 // streaming loads
+};
+
+template <class F, class T, class TO, int PL, int TL, int BS, bool NTS>
+__global__ __launch_bounds__(BS) void k_binary_transpose(const T* __restrict__ x, const T* __restrict__ y,
+                                                         TO* __restrict__ c, BinTransposeArgs ta, F f) {
+  constexpr int V = tr_vec<T>();
+  constexpr int TP = tr_tp<T, PL>();
+  constexpr int RP = BS / PL, NRP = TL / RP;    // L rows per read pass, read passes
+  constexpr int LPW = TL / V;                   // lanes along one output row
+  constexpr int WP = BS / LPW, NWP = TP / WP;   // P rows per write pass, write passes
+  static_assert(BS % PL == 0 && TL % RP == 0 && BS % LPW == 0 && TP % WP == 0, "passes must tile");
+  __shared__ T tile[TL][TP + 1];
+  const uint32_t id = blockIdx.x;
+  const uint32_t bq = fd_div(ta.tilesL, id);
+  const uint32_t tl = id - bq * ta.tilesL.d;
+  const uint32_t batch = fd_div(ta.tilesP, bq);
+  const uint32_t tp = bq - batch * ta.tilesP.d;
+  int64_t off[3];
+  row_offsets<3>(ta.batch, batch, off);
+  const uint64_t p0 = uint64_t(tp) * TP, l0 = uint64_t(tl) * TL;
+  const T* xb = x + off[1];
+  const T* yb = y + off[2];
+  TO* cb = c + off[0];
+  const int t = threadIdx.x;
+  const int pp = (t % PL) * V, lr = t / PL;     // read side
+  const int ll = (t % LPW) * V, pr = t / LPW;   // write side
+  const uint64_t l = l0 + ll;
+  Vec<T, V> yv[NWP];
+  if (l0 + TL <= ta.L && p0 + TP <= ta.P) {
+    Vec<T, V> xv[NRP];
+#pragma unroll
+    for (int k = 0; k < NRP; ++k)
+      xv[k] = vload_el_pol<T, V>(xb + int64_t(l0 + lr + k * RP) * ta.x_sL + int64_t(p0 + pp), ta.nt);
+    if (ta.y_unit) {
+#pragma unroll
+      for (int k = 0; k < NWP; ++k)
+        yv[k] = vload_el_pol<T, V>(yb + int64_t(p0 + pr + k * WP) * ta.y_sP + int64_t(l), ta.nt);
+    } else {
+#pragma unroll
+      for (int k = 0; k < NWP; ++k) {
+        const T s = yb[int64_t(p0 + pr + k * WP) * ta.y_sP];
+#pragma unroll
+        for (int q = 0; q < V; ++q) yv[k].v[q] = s;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NRP; ++k)
+#pragma unroll
+      for (int q = 0; q < V; ++q) tile[lr + k * RP][pp + q] = xv[k].v[q];
+  } else {
+    const uint64_t p = p0 + pp;
+    Vec<T, V> xv[NRP];
+#pragma unroll
+    for (int k = 0; k < NRP; ++k) {
+      const uint64_t r = l0 + lr + k * RP;
+      if (r >= ta.L) continue;
+      const T* src = xb + int64_t(r) * ta.x_sL + int64_t(p);
+      if (p + V <= ta.P) {
+        xv[k] = vload_el_pol<T, V>(src, ta.nt);
+      } else {
+#pragma unroll
+        for (int q = 0; q < V; ++q)
+          if (p + q < ta.P) xv[k].v[q] = src[q];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NWP; ++k) {
+      const uint64_t r = p0 + pr + k * WP;
+      if (r >= ta.P || l >= ta.L) continue;
+      const T* src = yb + int64_t(r) * ta.y_sP;
+      if (!ta.y_unit) {
+        const T s = src[0];
+#pragma unroll
+        for (int q = 0; q < V; ++q) yv[k].v[q] = s;
+      } else if (l + V <= ta.L) {
+        yv[k] = vload_el_pol<T, V>(src + l, ta.nt);
+      } else {
+#pragma unroll
+        for (int q = 0; q < V; ++q)
+          if (l + q < ta.L) yv[k].v[q] = src[l + q];
+      }
+    }
+    // lanes outside the array store unspecified values, which no lane inside it reads back
+#pragma unroll
+    for (int k = 0; k < NRP; ++k)
+#pragma unroll
+      for (int q = 0; q < V; ++q) tile[lr + k * RP][pp + q] = xv[k].v[q];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NWP; ++k) {
+    const uint64_t r = p0 + pr + k * WP;
+    if (r >= ta.P || l >= ta.L) continue;
+    TO* dst = cb + int64_t(r) * ta.out_sP + int64_t(l);
+    Vec<TO, V> v;
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      const T xe = tile[ll + q][pr + k * WP], ye = yv[k].v[q];
+      v.v[q] = ta.swap ? f(ye, xe) : f(xe, ye);
+    }
+    if (l + V <= ta.L) {
+      vstore_el<NTS, TO, V>(dst, v);
+    } else {
+#pragma unroll
+      for (int q = 0; q < V; ++q)
+        if (l + q < ta.L) dst[q] = v.v[q];
+    }
+  }
+}
+
+template <class F, class T, class TO, int PL, int TL, int BS, bool NTS>
+bool launch_binary_transpose_tiles(const T* x, const T* y, TO* c, BinTransposeArgs ta, uint64_t nb, hipStream_t st,
+                                   F f) {
+  const uint64_t tL = (ta.L + TL - 1) / TL, tP = (ta.P + tr_tp<T, PL>() - 1) / tr_tp<T, PL>();
+  if (tL * tP * nb >= (uint64_t(1) << 31)) return false;
+  ta.tilesL = make_fastdiv(uint32_t(tL));
+  ta.tilesP = make_fastdiv(uint32_t(tP));
+  k_binary_transpose<F, T, TO, PL, TL, BS, NTS><<<dim3(unsigned(tL * tP * nb)), BS, 0, st>>>(x, y, c, ta, f);
+  return true;
+}
+
+// false when the operands do not have this form; nothing is launched then
+template <class F, class T, class TO>
+bool launch_binary_transpose(const T* a, const T* b, TO* c, const Plan& p, bool nt, bool nts, hipStream_t st, F f) {
+  const int nd = p.ndim;
+  if (nd < 2) return false;
+  for (int o = 1; o <= 2; ++o) {
+    const int64_t xs = p.stride[o][nd - 1], ys = p.stride[3 - o][nd - 1];
+    if (xs == 0 || xs == 1 || xs == -1 || (ys != 0 && ys != 1)) continue;
+    int P = -1;
+    for (int d = nd - 2; d >= 0 && P < 0; --d)
+      if (p.stride[o][d] == 1) P = d;
+    if (P < 0) continue;
+    BinTransposeArgs ta{};
+    ta.P = p.shape[P];
+    ta.L = p.shape[nd - 1];
+    if (ta.P < kBinTransposeMin || ta.L < kBinTransposeMin || ta.P >= (uint64_t(1) << 32) ||
+        ta.L >= (uint64_t(1) << 32))
+      continue;
+    ta.x_sL = xs;
+    ta.y_sP = p.stride[3 - o][P];
+    ta.y_unit = ys == 1;
+    ta.out_sP = p.stride[0][P];
+    ta.swap = o == 2;
+    ta.nt = nt;
+    const uint64_t nb = p.numel / (ta.P * ta.L);
+    bool fits = true;
+    for (int d = nd - 2; d >= 0; --d) {
+      if (d == P) continue;
+      if (p.shape[d] >= (uint64_t(1) << 32)) fits = false;
+      const int k = ta.batch.nd++;
+      ta.batch.div[k] = make_fastdiv(uint32_t(p.shape[d]));
+      ta.batch.stride[0][k] = p.stride[0][d];
+      ta.batch.stride[1][k] = p.stride[o][d];
+      ta.batch.stride[2][k] = p.stride[3 - o][d];
+    }
+    if (!fits) continue;
+    const T* x = o == 1 ? a : b;
+    const T* y = o == 1 ? b : a;
+    if (ta.L <= 32) return launch_binary_transpose_tiles<F, T, TO, 64, 32, 512, false>(x, y, c, ta, nb, st, f);
+    if (ta.L <= 64 || ta.P <= 64 || p.numel < kBinTransposeSmall)
+      return launch_binary_transpose_tiles<F, T, TO, 8, 64, 256, false>(x, y, c, ta, nb, st, f);
+    if (nts) return launch_binary_transpose_tiles<F, T, TO, 32, 128, 1024, true>(x, y, c, ta, nb, st, f);
+    return launch_binary_transpose_tiles<F, T, TO, 32, 128, 1024, false>(x, y, c, ta, nb, st, f);
+  }
+  return false;
+}
+
+// ---------------------------------------------------------------------------------------------
 // generic fallback: 64-bit decode per element (shapes beyond the 32-bit row limits).
 struct NdMeta64 {
   int nd;
@@ -710,6 +908,7 @@ void launch_binary(const T* a, const T* b, TO* c, int ndim, const size_t* shape,
     });
     return;
   }
+  if (launch_binary_transpose<F, T, TO>(a, b, c, p, nt, nts, st, f)) return;
   if (rows_ok(p, V)) {
     const uint32_t L = uint32_t(p.shape[nd - 1]);
     const int64_t sa = p.stride[1][nd - 1], sb = p.stride[2][nd - 1];
