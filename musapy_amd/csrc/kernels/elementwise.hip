@@ -441,7 +441,7 @@ bool launch_transpose_tiles(const TI* a, TO* c, TransposeArgs ta, uint64_t nb, b
   constexpr uint64_t TP = tr_tp<TI, PL>();
   constexpr int TL = tr_tl<TO, TI, PL, BS, ROWS>();
   const uint64_t tL = (ta.L + TL - 1) / TL, tP = (ta.P + TP - 1) / TP;
-  if (tL * tP * nb >= (uint64_t(1) << 31)) return false;
+  if (!grid_fits(tL * tP * nb, BS)) return false;
   ta.tilesL = make_fastdiv(uint32_t(tL));
   ta.tilesP = make_fastdiv(uint32_t(tP));
   with_store_policy(nts, [&](auto NT) {
@@ -624,7 +624,7 @@ template <class F, class T, class TO, int PL, int TL, int BS, bool NTS>
 bool launch_binary_transpose_tiles(const T* x, const T* y, TO* c, BinTransposeArgs ta, uint64_t nb, hipStream_t st,
                                    F f) {
   const uint64_t tL = (ta.L + TL - 1) / TL, tP = (ta.P + tr_tp<T, PL>() - 1) / tr_tp<T, PL>();
-  if (tL * tP * nb >= (uint64_t(1) << 31)) return false;
+  if (!grid_fits(tL * tP * nb, BS)) return false;
   ta.tilesL = make_fastdiv(uint32_t(tL));
   ta.tilesP = make_fastdiv(uint32_t(tP));
   k_binary_transpose<F, T, TO, PL, TL, BS, NTS><<<dim3(unsigned(tL * tP * nb)), BS, 0, st>>>(x, y, c, ta, f);
@@ -925,7 +925,7 @@ void launch_binary(const T* a, const T* b, TO* c, int ndim, const size_t* shape,
       const uint32_t groups = (L + uint32_t(kPieceBlock) * V * U - 1) / (uint32_t(kPieceBlock) * V * U);
       ra.groups = make_fastdiv(groups);
       const uint64_t blocks = uint64_t(p.numel / L) * groups;
-      if (blocks < (uint64_t(1) << 31)) {
+      if (grid_fits(blocks, kPieceBlock)) {
         with_store_policy(nts, [&](auto NT) {
           k_binary_rowpieces<V, U, NT.value, F, T, TO><<<dim3(unsigned(blocks)), kPieceBlock, 0, st>>>(ia, sa, ib, sb,
                                                                                                        c, ra, f);

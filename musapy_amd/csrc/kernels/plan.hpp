@@ -39,6 +39,12 @@ inline uint32_t fd_div_host(const FastDiv& f, uint32_t n) {
   return uint32_t((uint64_t(t) + n) >> f.s);
 }
 
+// Whether a launch of `blocks` blocks of `lanes` lanes is accepted: HIP counts a grid dim in lanes, below
+// 2^32, and block ids are decoded as positive 32-bit numbers here.
+inline bool grid_fits(uint64_t blocks, uint64_t lanes) {
+  return blocks < (uint64_t(1) << 31) && blocks * lanes < (uint64_t(1) << 32);
+}
+
 // Elementwise plan.  Operand 0 is the (C-contiguous) output, operands 1.. are inputs.
 struct Plan {
   int nops;

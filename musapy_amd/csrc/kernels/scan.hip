@@ -815,7 +815,7 @@ ColScanRoute col_scan_route(const ScanPlan& p) {
   const uint64_t TR = uint64_t(claim ? kColBlockClaim : kColBlock) / (thin ? kColLpcThin : kColLpc) * kColRpl;
   const uint64_t tiles = (p.L + TR - 1) / TR;
   const uint64_t per = claim ? groups : (groups + 7) / 8 * 8;
-  if (per * tiles >= (uint64_t(1) << 31)) return r;
+  if (!grid_fits(per * tiles, claim ? kColBlockClaim : kColBlock)) return r;
   r.kind = ColScanRoute::kTiles;
   r.strips = uint32_t(strips);
   r.groups = uint32_t(groups);

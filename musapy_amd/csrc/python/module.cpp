@@ -627,6 +627,7 @@ PYBIND11_MODULE(_core, m) {
     }
     return py::make_tuple(r.shape, r.strides, r.offset);
   });
+  m.def("_grid_fits", [](uint64_t blocks, uint64_t lanes) { return mpy::grid_fits(blocks, lanes); });
   m.def("_plan_elementwise", [](const Shape& shape, const std::vector<Strides>& ins) {
     mpy::Plan p{};
     std::vector<const ssize_t*> ptrs;

@@ -128,6 +128,16 @@ def test_scan_plan_kinds():
     assert _core._plan_scan([8, 9], [1, 8], 1)["kind"] == "generic"
 
 
+def test_grid_limits():
+    """A grid dim holds fewer than 2^32 lanes, whatever the block size, and fewer than 2^31 blocks."""
+    for lanes in (64, 128, 256, 512, 1024):
+        most = min(2 ** 31 - 1, (2 ** 32 - 1) // lanes)
+        assert _core._grid_fits(1, lanes) and _core._grid_fits(most, lanes)
+        assert not _core._grid_fits(most + 1, lanes)
+    assert not _core._grid_fits(8400000, 512)  # 16 x 16 transposed batches, one tile of 512 lanes each
+    assert not _core._grid_fits(32768 * 128, 1024)  # cumsum of (32768, 262144, 2) along axis 1 in 2048-row tiles
+
+
 def test_fastdiv_exact():
     rng = np.random.default_rng(5)
     divisors = [1, 2, 3, 5, 7, 10, 31, 64, 641, 1000, 4096, 6700417, 2**31 - 1, 2**31, 2**31 + 1, 2**32 - 1]
