@@ -446,7 +446,9 @@ uint32_t musapy_kernels_set_spin_limit(uint32_t polls);
 
 /* ---- planning helper (new; no counterpart in kernels.rs) ----
  * Tiles per output that the partial entry points should be given for this reduction on this
- * device: 1 means a single-pass entry point already fills the GPU. */
+ * device: 1 means a single-pass entry point already fills the GPU.  _v2 answers for one `op`
+ * (MUSAPY_RED_*) in the compute dtype `dtype`, the other form for whichever op wants more. */
+size_t musapy_reduce_tiles_hint_v2(int op, int dtype, int ndim, const size_t* in_shape, const ssize_t* in_strides, int axis, size_t axis_len, size_t out_size);
 size_t musapy_reduce_tiles_hint(int ndim, const size_t* in_shape, const ssize_t* in_strides, int axis, size_t axis_len, size_t out_size, size_t elem_size);
 
 #ifdef __cplusplus

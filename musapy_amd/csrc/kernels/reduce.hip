@@ -154,13 +154,22 @@ inline int fused_dispatch(int op, int dtype, const void* a, void* c, int ndim, c
 
 extern "C" {
 
-size_t musapy_reduce_tiles_hint(int ndim, const size_t* in_shape, const ssize_t* in_strides, int axis,
-                                size_t axis_len, size_t out_size, size_t elem_size) {
-  if (out_size == 0 || axis_len == 0) return 1;
+static size_t hint(RedKind kind, RED_ARGS, size_t elem_size) {
+  if (out_size == 0 || axis_len == 0 || elem_size == 0) return 1;
   if (ndim < 0 || ndim > kMaxDims || (ndim > 0 && (axis < 0 || axis >= ndim))) return 1;  // the launch reports it
   ReducePlan p;
-  plan_reduce(p, ndim, in_shape, in_strides, axis, axis_len, out_size);
-  return tiles_hint(p, elem_size);
+  plan_reduce(p, RED_PASS);
+  return tiles_hint(p, elem_size, kind);
+}
+size_t musapy_reduce_tiles_hint_v2(int op, int dtype, RED_ARGS) {
+  const bool sum = op == MUSAPY_RED_SUM || op == MUSAPY_RED_PROD || op == MUSAPY_RED_MEAN;
+  const bool cplx = dtype == MUSAPY_DT_C64 || dtype == MUSAPY_DT_C128;
+  const size_t es = dtype == MUSAPY_DT_C128 ? 16 : dtype == MUSAPY_DT_F32 ? 4 : 8;
+  return hint(!sum ? RedKind::kOrdered : cplx ? RedKind::kComplexSum : RedKind::kSum, RED_PASS, es);
+}
+size_t musapy_reduce_tiles_hint(RED_ARGS, size_t elem_size) {
+  const size_t sum = hint(RedKind::kSum, RED_PASS, elem_size), ext = hint(RedKind::kOrdered, RED_PASS, elem_size);
+  return sum > ext ? sum : ext;
 }
 
 // value reductions whose final step is the plain accumulator (sum/prod/max/min, real + complex)

@@ -82,7 +82,7 @@ IntRoute int_route(const ReducePlan& p, size_t es, uint32_t V) {
     return r;
   }
   // row segments: as tiles_hint, for segments of at least 32 KB
-  if (p.out_size < 2048 && p.out_size * p.R * es > (uint64_t(256) << 10)) {
+  if (p.out_size < 2048 && p.out_size * p.R * es > (uint64_t(128) << 10)) {
     uint64_t tiles = ceil_div(uint64_t(4096), p.out_size);
     const uint64_t most = ceil_div(p.R * es, 32768);
     r.tiles = size_t(tiles < most ? tiles : most);
@@ -141,7 +141,8 @@ int run_int(const void* av, RedOut<O> out, const IntCall& c) {
   if (r.kind == IntRoute::kLanes) {
     const uint32_t vpr = uint32_t(ceil_div(C, V));
     const uint32_t items = uint32_t(p.out_size / C * vpr);
-    k_reduce_lane<Op, T, V, kSpanUnroll, S, O><<<dim3(unsigned(ceil_div(items, kRBlock))), kRBlock, 0, c.st>>>(
+    const uint32_t bs = lane_block(items);
+    k_reduce_lane<Op, T, V, kSpanUnroll, S, O><<<dim3(unsigned(ceil_div(items, bs))), bs, 0, c.st>>>(
         a, out_indexer(p, p.ond - 1), uint32_t(C), make_fastdiv(vpr), p.R, p.rstride, items, out);
     return 0;
   }

@@ -19,6 +19,7 @@
 
 #include "kcommon.hpp"
 #include "reduce_ops.hpp"
+#include "routes.hpp"
 #include "publish.hpp"
 #include "../../../include/musapy_kernels.h"
 
@@ -850,27 +851,23 @@ struct SpanArgs {
   int64_t rs;
   bool flat;           // rows are contiguous (rs == C, one strip): a vector may run into the next row
 };
-constexpr int kSpanBS = 512;
-constexpr int kSpanUnroll = 8;
-
-// Accumulators that a lane keeps per column: one per row in flight where sums round in the element's
-// own type, so that the chain of additions behind a column is an eighth of the lane's rows, as when the
-// 8 waves of the column kernel share them; one otherwise (ordered and integer results are exact, and
-// c64 sums run in 64 bits).  One accumulator for all rows measured an error against 64 bits of 3.6e-7
-// for f32 sums over 572 rows; the column kernel has 6.7e-8.
+// Sums that round in the element's own type (ordered and integer results are exact, and c64 sums run in
+// 64 bits).  The column kernel's 8 waves share the rows of such a sum; a single accumulator for all of
+// them measured an error against 64 bits of 3.6e-7 for f32 sums over 572 rows, where that kernel has
+// 6.7e-8.  So the lane kernel keeps one accumulator per row in flight and joins them as a tree, and the
+// span kernel, whose m rows per step are spread over lanes already, adds its 8 rows in flight as a tree
+// before they meet the accumulator (accumulators of their own would cost it the second block per CU).
 template <class Op, class T>
-constexpr int col_accs(int unroll) {
-  return !Op::kOrdered && std::is_same_v<typename Op::A, T> ? unroll : 1;
+constexpr bool rounds_in_type() {
+  return !Op::kOrdered && std::is_same_v<typename Op::A, T>;
 }
-// joins them into the first, as a tree
-template <class Op, int N, int VEC>
-__device__ inline void join_accs(typename Op::A (&acc)[N][VEC]) {
+template <class Op, int N>
+__device__ inline typename Op::A tree_fold(typename Op::A (&t)[N]) {
 #pragma unroll
   for (int h = N / 2; h > 0; h /= 2)
 #pragma unroll
-    for (int u = 0; u < h; ++u)
-#pragma unroll
-      for (int v = 0; v < VEC; ++v) acc[u][v] = Op::comb(acc[u][v], acc[u + h][v]);
+    for (int u = 0; u < h; ++u) t[u] = Op::comb(t[u], t[u + h]);
+  return t[0];
 }
 
 template <class Op, class T, int VEC, int UNROLL, bool FINAL, class S = T, class O = T>
@@ -896,13 +893,11 @@ __global__ __launch_bounds__(kSpanBS) void k_reduce_span(const S* __restrict__ a
   // shares with its neighbour get the same values twice)
   const int32_t shift = !sa.flat && cbase + c0 + VEC > sa.C ? int32_t(cbase + c0 + VEC - sa.C) : 0;
   const uint32_t step_rows = sa.m * UNROLL;
-  constexpr int kAcc = col_accs<Op, T>(UNROLL);
-  A acc[kAcc][VEC];
+  A acc[VEC];
   uint32_t rv[VEC];                     // row of element v inside a step
 #pragma unroll
   for (int v = 0; v < VEC; ++v) {
-#pragma unroll
-    for (int u = 0; u < kAcc; ++u) acc[u][v] = Op::init();
+    acc[v] = Op::init();
     rv[v] = sa.flat ? (e + v) / sa.cw : r0;
   }
   if (live) {
@@ -913,6 +908,8 @@ __global__ __launch_bounds__(kSpanBS) void k_reduce_span(const S* __restrict__ a
       const S* q = lp + int64_t((uint64_t(t) + k * sa.tiles) * step_rows) * sa.rs;
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) d[u] = vload_el<S, VEC>(q + int64_t(uint64_t(u) * sa.m) * sa.rs);
+      // (the scheduler would move some of these loads below the tree of the round before)
+      if constexpr (rounds_in_type<Op, T>()) __builtin_amdgcn_sched_barrier(0);
     };
     auto fold = [&](uint64_t k, const Vec<S, VEC>(&src)[UNROLL]) {
       const uint32_t row = uint32_t((uint64_t(t) + k * sa.tiles) * step_rows);
@@ -921,11 +918,13 @@ __global__ __launch_bounds__(kSpanBS) void k_reduce_span(const S* __restrict__ a
         T xs[UNROLL][1];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) xs[u][0] = T(src[u].v[v]);
-        if constexpr (kAcc == 1) {
-          acc[0][v] = Op::template step_chunk<UNROLL, 1>(acc[0][v], xs, row + rv[v], sa.m);
-        } else {
+        if constexpr (rounds_in_type<Op, T>()) {
+          A t[UNROLL];
 #pragma unroll
-          for (int u = 0; u < UNROLL; ++u) acc[u % kAcc][v] = Op::step(acc[u % kAcc][v], xs[u][0], 0);
+          for (int u = 0; u < UNROLL; ++u) t[u] = xs[u][0];
+          acc[v] = Op::comb(acc[v], tree_fold<Op>(t));
+        } else {
+          acc[v] = Op::template step_chunk<UNROLL, 1>(acc[v], xs, row + rv[v], sa.m);
         }
       }
     };
@@ -943,27 +942,42 @@ __global__ __launch_bounds__(kSpanBS) void k_reduce_span(const S* __restrict__ a
         const S* q = row + rv[VEC - 1] < sa.R ? lp + int64_t(row) * sa.rs : safe;
         x[u] = vload_el<S, VEC>(q);
       }
+      constexpr bool kTree = rounds_in_type<Op, T>();
+      A ts[kTree ? VEC : 1][UNROLL];
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
         const uint64_t row = base + uint64_t(u) * sa.m;
+        if constexpr (kTree) {
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) ts[v][u] = Op::init();
+        }
         if (row + rv[VEC - 1] < sa.R) {
 #pragma unroll
-          for (int v = 0; v < VEC; ++v) acc[u % kAcc][v] = Op::step(acc[u % kAcc][v], T(x[u].v[v]), int64_t(row + rv[v]));
+          for (int v = 0; v < VEC; ++v) {
+            if constexpr (kTree) ts[v][u] = T(x[u].v[v]);
+            else acc[v] = Op::step(acc[v], T(x[u].v[v]), int64_t(row + rv[v]));
+          }
         } else if (row + rv[0] < sa.R) {  // the vector that the end of the slice cuts (flat rows)
           const S* q = lp + int64_t(row) * sa.rs;
 #pragma unroll
           for (int v = 0; v < VEC; ++v)
-            if (row + rv[v] < sa.R) acc[u % kAcc][v] = Op::step(acc[u % kAcc][v], T(q[v]), int64_t(row + rv[v]));
+            if (row + rv[v] < sa.R) {
+              if constexpr (kTree) ts[v][u] = T(q[v]);
+              else acc[v] = Op::step(acc[v], T(q[v]), int64_t(row + rv[v]));
+            }
         }
       }
+      if constexpr (kTree) {
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) acc[v] = Op::comb(acc[v], tree_fold<Op>(ts[v]));
+      }
     }
-    join_accs<Op, kAcc, VEC>(acc);
   }
   // the m x cw accumulators of the block, in row-major order
   if (live) {
 #pragma unroll
     for (int v = 0; v < VEC; ++v)
-      if (shift <= int32_t(c0) + v || sa.flat) s[int32_t(e) - shift + v] = acc[0][v];
+      if (shift <= int32_t(c0) + v || sa.flat) s[int32_t(e) - shift + v] = acc[v];
   }
   __syncthreads();
   for (uint32_t rows = sa.m; rows > 1;) {
@@ -1048,11 +1062,11 @@ __global__ __launch_bounds__(kSpanBS) void k_span_final(const S* __restrict__ a,
 // LDS, no second level.  The last vector of a row is moved back to end with the row: its columns
 // are computed twice, with the same result.
 template <class Op, class T, int VEC, int UNROLL, class S = T, class O = T>
-__global__ __launch_bounds__(kRBlock) void k_reduce_lane(const S* __restrict__ a, RowIndexer<1> ix, uint32_t C,
+__global__ __launch_bounds__(kLaneBS) void k_reduce_lane(const S* __restrict__ a, RowIndexer<1> ix, uint32_t C,
                                                          FastDiv vpr, uint64_t R, int64_t rs, uint32_t items,
                                                          RedOut<O> out) {
   using A = typename Op::A;
-  const uint32_t g = blockIdx.x * kRBlock + threadIdx.x;
+  const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= items) return;
   const uint32_t outer = fd_div(vpr, g);
   uint32_t c0 = (g - outer * vpr.d) * VEC;
@@ -1060,7 +1074,7 @@ __global__ __launch_bounds__(kRBlock) void k_reduce_lane(const S* __restrict__ a
   int64_t off[1];
   row_offsets<1>(ix, outer, off);
   const S* p = a + off[0] + c0;
-  constexpr int kAcc = col_accs<Op, T>(UNROLL);
+  constexpr int kAcc = rounds_in_type<Op, T>() ? UNROLL : 1;
   A acc[kAcc][VEC];
   T first[VEC];
 #pragma unroll
@@ -1079,6 +1093,7 @@ __global__ __launch_bounds__(kRBlock) void k_reduce_lane(const S* __restrict__ a
     Vec<S, VEC> x[UNROLL];
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) x[u] = vload_el<S, VEC>(p + int64_t(k + u) * rs);
+    if constexpr (rounds_in_type<Op, T>()) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int v = 0; v < VEC; ++v) {
       T xs[UNROLL][1];
@@ -1104,10 +1119,12 @@ __global__ __launch_bounds__(kRBlock) void k_reduce_lane(const S* __restrict__ a
         acc[u % kAcc][v] = Op::step(acc[u % kAcc][v], T(x[u].v[v]), int64_t(k + u));
     }
   }
-  join_accs<Op, kAcc, VEC>(acc);
 #pragma unroll
   for (int v = 0; v < VEC; ++v) {
-    A r = acc[0][v];
+    A t[kAcc];
+#pragma unroll
+    for (int u = 0; u < kAcc; ++u) t[u] = acc[u][v];
+    A r = tree_fold<Op>(t);
     if constexpr (Op::kOrdered) r = absorb_first<Op, T>(r, first[v]);
     write_result<Op, T, kWriteFinal, O>(out, uint64_t(outer) * C + c0 + v, r, 0);
   }
@@ -1662,8 +1679,6 @@ __global__ __launch_bounds__(kRBlock) void k_reduce_pairs(const T* __restrict__ 
 
 // ============================================================================================
 // host side
-inline uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
-
 template <class T> constexpr int rvec() { return sizeof(T) >= 16 ? 1 : int(16 / sizeof(T)); }
 
 inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -1680,93 +1695,18 @@ inline RowIndexer<1> out_indexer(const ReducePlan& p, int ndims) {
   return ix;
 }
 
-// How a column reduction (strided axis, unit-stride outputs) runs:
-//  * lanes, when one lane per 16 bytes of outputs makes at least 32768 lanes (two waves per CU):
-//    (512, 16, 2048) f32 over axis 1: max 24.5 -> 13.7 us, sum 14.7 -> 13.6;
-//  * spans, for rows of up to 4 KB (sums) or less than 4 KB (max / min / arg) that a block of at most
-//    512 lanes can cover with a whole number of rows per step.  256 blocks (one per CU, 8 x 16-byte
-//    loads in flight per lane, twice buffered) ran faster than 512 and 1024: (1000003, 37) f32 mean
-//    444 (column kernel) -> 30.8 us, against 32.8 and 36.2; max 941 -> 33.8; (131072, 384) f32 mean
-//    55.9 -> 36, against 45.7 with 512.  Rows of exactly 4 KB: (32768, 1024) f32 mean 38.3 -> 28.8 us,
-//    but max 29.8 -> 31.4.  Inputs of at most 4 MB split by column strips instead of row tiles, which
-//    saves the second launch ((300, 700) f32 sum 6.7 -> 4.4 us, 6.8 with row tiles; at 25 MB the
-//    strips' short runs cost more than the launch: (64, 1000, 100) 14.1 against 10.4 us);
-//  * the 64-lane column kernel otherwise.
-struct ColRoute {
-  enum : int { kColumns = 0, kLanes = 1, kSpans = 2 };
-  int kind = kColumns;
-  uint32_t bs = 0, cw = 0, strips = 1, m = 0, lanes = 0, tiles = 1;
-  bool flat = false;
-};
-constexpr uint64_t kLaneItems = 32768;
-constexpr uint64_t kSpanRowBytes = 4096;
-constexpr uint64_t kSpanBlocks = 256;
-constexpr uint64_t kSpanStripBytes = uint64_t(4) << 20;
-
-inline uint32_t gcd32(uint32_t a, uint32_t b) { return b == 0 ? a : gcd32(b, a % b); }
-
-inline ColRoute col_route(const ReducePlan& p, size_t es, bool ordered) {
-  ColRoute r;
-  const uint32_t V = es >= 16 ? 1 : uint32_t(16 / es);
-  const uint64_t C = p.oshape[p.ond - 1];
-  const uint64_t outer = p.out_size / C;
-  if (p.kind != kColReduce || p.R >= (uint64_t(1) << 31) || C >= (uint64_t(1) << 31)) return r;
-  // the outer dims are decoded in 32 bits
-  if (outer >= (uint64_t(1) << 31)) return r;
-  const uint64_t items = outer * ceil_div(C, V);
-  if (C >= V && items >= kLaneItems && items < (uint64_t(1) << 31)) {
-    r.kind = ColRoute::kLanes;
-    return r;
-  }
-  if (C * es > kSpanRowBytes || (ordered && C * es == kSpanRowBytes)) return r;
-  const bool contiguous = p.rstride == int64_t(C);
-  if ((C % V != 0 && !contiguous) || p.R * C < V) return r;
-  const uint64_t round = uint64_t(kSpanBS) * kSpanUnroll * V;  // elements of one round of a whole block
-  uint64_t cw = C;
-  if (C % V == 0 && outer < kSpanBlocks && p.R * C > round && outer * p.R * C * es <= kSpanStripBytes) {
-    cw = C / ceil_div(kSpanBlocks, outer) / V * V;
-    const uint64_t least = 64 / es;  // 64-byte runs
-    if (cw < least) cw = least;
-    if (cw > C) cw = C;
-  }
-  const uint32_t period = uint32_t(cw) / gcd32(uint32_t(cw), V);  // lanes of the shortest whole-row step
-  if (period > uint32_t(kSpanBS)) return r;
-  r.cw = uint32_t(cw);
-  r.strips = uint32_t(ceil_div(C, cw));
-  if (outer * r.strips * kSpanBlocks >= (uint64_t(1) << 31)) return r;
-  r.kind = ColRoute::kSpans;
-  r.flat = contiguous && r.strips == 1;
-  // the block size with the fewest idle lanes, no larger than one round of the slice needs
-  uint64_t most = ceil_div(ceil_div(p.R * cw, uint64_t(V) * kSpanUnroll), kWave) * kWave;
-  const uint64_t least = ceil_div(period, kWave) * kWave;
-  if (most < least) most = least;
-  if (most > uint64_t(kSpanBS)) most = kSpanBS;
-  for (uint32_t bs = uint32_t(most); bs >= least && 2 * bs > most; bs -= kWave) {
-    const uint32_t n = bs / period * period;
-    if (r.bs == 0 || uint64_t(n) * r.bs > uint64_t(r.lanes) * bs + uint64_t(r.bs) * bs / 50) {
-      r.bs = bs;
-      r.lanes = n;
-    }
-  }
-  r.m = uint32_t(uint64_t(r.lanes) * V / cw);
-  // a second launch folds the tiles: not worth it below 6 rounds
-  const uint64_t chunks = p.R / (uint64_t(r.m) * kSpanUnroll);
-  uint64_t tiles = ceil_div(kSpanBlocks, outer * r.strips);
-  if (tiles > chunks / 2) tiles = chunks / 2;
-  // the partials (at most 2 * es bytes each) have to fit the 1 MiB workspace of a stream
-  const uint64_t room = (uint64_t(1) << 20) / (p.out_size * 2 * es);
-  if (tiles > room) tiles = room;
-  r.tiles = uint32_t(chunks < 6 || tiles < 1 ? 1 : tiles);
-  return r;
+template <class Op, class T>
+constexpr RedKind red_kind() {
+  return Op::kOrdered ? RedKind::kOrdered
+         : std::is_same_v<T, c64> || std::is_same_v<T, c128> ? RedKind::kComplexSum : RedKind::kSum;
 }
 
 // Recommended tiles per output: enough (output, tile) work items to fill 256 CUs several times
 // over while each tile still streams a few tens of KB.
-inline size_t tiles_hint(const ReducePlan& p, size_t es) {
+inline size_t tiles_hint(const ReducePlan& p, size_t es, RedKind kind) {
   if (p.R <= 1 || p.out_size == 0) return 1;
   if (p.kind == kColReduce) {
-    // (rows of exactly 4 KB, where sums and ordered ops part, take the column kernel's tiles here)
-    const ColRoute route = col_route(p, es, true);
+    const ColRoute route = col_route(p, es, kind);
     if (route.kind == ColRoute::kLanes) return 1;
     if (route.kind == ColRoute::kSpans) return route.tiles;
     // column tiles: ~256 long-lived blocks (one per CU, 8 loads of 16 bytes in flight per lane)
@@ -1927,12 +1867,13 @@ void launch_reduce(const T* a, RedOut<T> out, int ndim, const size_t* shape, con
   constexpr int V = rvec<T>();
   if constexpr (WRITE == kWriteFinal) {
     if (tiles == 1 && p.R > 0) {
-      const ColRoute r = col_route(p, sizeof(T), Op::kOrdered);
+      const ColRoute r = col_route(p, sizeof(T), red_kind<Op, T>());
       if (r.kind == ColRoute::kLanes) {
         const uint32_t C = uint32_t(p.oshape[p.ond - 1]);
         const uint32_t vpr = uint32_t(ceil_div(C, V));
         const uint32_t items = uint32_t(p.out_size / C * vpr);
-        k_reduce_lane<Op, T, V, kSpanUnroll><<<dim3(unsigned(ceil_div(items, kRBlock))), kRBlock, 0, st>>>(
+        const uint32_t bs = lane_block(items);
+        k_reduce_lane<Op, T, V, kSpanUnroll><<<dim3(unsigned(ceil_div(items, bs))), bs, 0, st>>>(
             a, out_indexer(p, p.ond - 1), C, make_fastdiv(vpr), p.R, p.rstride, items, out);
         return;
       }
@@ -2092,7 +2033,7 @@ int launch_reduce_fused(const T* a, RedOut<T> out, int ndim, const size_t* shape
   ReducePlan p;
   plan_reduce(p, ndim, shape, strides, axis, axis_len, out_size);
   if (p.kind == kColReduce) {
-    const ColRoute r = col_route(p, sizeof(T), Op::kOrdered);
+    const ColRoute r = col_route(p, sizeof(T), red_kind<Op, T>());
     if (r.kind == ColRoute::kLanes) {
       launch_reduce<Op, T, kWriteFinal>(a, out, ndim, shape, strides, axis, axis_len, out_size, 1, st);
       return kFusedLaunched;

@@ -1,0 +1,147 @@
+// routes.hpp -- which kernel variant a launch takes, from its plan alone (pure C++, like plan.hpp).
+#pragma once
+
+#include "plan.hpp"
+
+namespace mpy {
+
+inline uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
+inline uint32_t gcd32(uint32_t a, uint32_t b) { return b == 0 ? a : gcd32(b, a % b); }
+
+// ---------------------------------------------------------------------------------------------
+// How a column reduction (strided axis, unit-stride outputs) runs.  Three kernels share the shapes;
+// the lines between them are those of a sweep over 1 to 20000 slices of 5 to 500000 rows of 8 to
+// 600000 columns (f32 and f64, sums and max), and every figure below is from it.  `vecs` counts the
+// 16-byte vectors of a row, `items` those of all slices.
+//  * lanes: one lane per vector walks the whole axis.  It needs many of them (65536 lanes are one wave
+//    per SIMD); then it is level with the column kernel or ahead of it, most where that one leaves lanes
+//    idle or has less than a round of rows: (20000, 16, 8) sum 44.6 -> 7.3 us, (1000, 16, 512) max 13.2
+//    -> 8.1.  With fewer the column kernel keeps more loads in flight ((256, 500, 512) max 44.8 against
+//    73 us), and rows that fill its lanes only in part want 262144: (4000, 100, 300) sum 99 -> 82 us,
+//    but (4000, 100, 100) 27 -> 32.
+//  * spans: a block reads a whole number of rows per step.  They pay where the column kernel's 64 lanes
+//    do not fill ((256, 4000, 8) sum 67.6 -> 9.1 us), or where one or a few slices leave it strips that
+//    are far apart in memory ((30000, 512) sum 32 -> 14); with many slices of full rows they only cost
+//    ((64, 100, 1000) sum 7.2 -> 14.6, (120, 2000, 1024) 145 -> 183).  Max / min / arg over one slice
+//    keep the column kernel unless the array is long: (4000, 128) 9.0 us, 16.3 by spans.
+//    Inputs of at most 4 MB split by column strips instead of row tiles, which saves the second
+//    launch, if a strip is at most one and a half rounds long: (600, 400) sum 7.3 -> 5.4 us, but (3000,
+//    100) 11.7 by columns, 13.7 by strips and 9.3 by tiles.
+//  * columns: the 64-lane column kernel, for everything else.
+struct ColRoute {
+  enum : int { kColumns = 0, kLanes = 1, kSpans = 2 };
+  int kind = kColumns;
+  uint32_t bs = 0, cw = 0, strips = 1, m = 0, lanes = 0, tiles = 1;
+  bool flat = false;
+};
+constexpr int kSpanBS = 512;
+constexpr int kSpanUnroll = 8;
+constexpr int kLaneBS = 256;
+constexpr uint64_t kLaneItems = 32768;
+// Lanes per block.  Blocks of 256 put a wave on each SIMD of their CU; where they leave a sparse second
+// round, single waves spread more evenly: (72, 300000) f32 sum, 75000 lanes, 18.6 -> 16.0 us; but (1000,
+// 200003), 50001 lanes, 119 -> 136 and (4000, 100, 300), 300000 lanes, 82 -> 90.
+inline uint32_t lane_block(uint64_t items) {
+  const uint64_t blocks = ceil_div(items, uint64_t(kLaneBS)), rounds = ceil_div(blocks, uint64_t(256));
+  return rounds > 1 && items < 6 * kLaneItems && 100 * blocks < 85 * 256 * rounds ? 64 : kLaneBS;
+}
+constexpr uint64_t kSpanRowBytes = 4096;
+constexpr uint64_t kSpanBlocks = 256;
+constexpr uint64_t kSpanStripBytes = uint64_t(4) << 20;
+
+// columns per strip of a small input, 0 for tiles along the rows
+inline uint64_t span_strip(uint64_t outer, uint64_t R, uint64_t C, uint64_t es, uint64_t V, uint64_t round) {
+  if (C % V != 0 || outer >= kSpanBlocks || R * C <= round || outer * R * C * es > kSpanStripBytes) return 0;
+  uint64_t cw = C / ceil_div(kSpanBlocks, outer) / V * V;
+  const uint64_t least = 64 / es;  // 64-byte runs
+  if (cw < least) cw = least;
+  return cw < C && 2 * R * cw <= 3 * round ? cw : 0;
+}
+
+enum class RedKind { kSum, kComplexSum, kOrdered };  // sum / prod / mean, of complex elements, max / min / arg
+
+inline ColRoute col_route(const ReducePlan& p, size_t es, RedKind kind) {
+  const bool ordered = kind == RedKind::kOrdered;
+  ColRoute r;
+  const uint32_t V = es >= 16 ? 1 : uint32_t(16 / es);
+  const uint64_t C = p.oshape[p.ond - 1], R = p.R;
+  const uint64_t outer = p.out_size / C;
+  if (p.kind != kColReduce || R >= (uint64_t(1) << 31) || C >= (uint64_t(1) << 31)) return r;
+  // the outer dims are decoded in 32 bits
+  if (outer >= (uint64_t(1) << 31)) return r;
+  const uint64_t vecs = ceil_div(C, V), groups = ceil_div(vecs, 64), items = outer * vecs;
+  const bool narrow = vecs <= 16;                     // a quarter of a column group's lanes at most
+  const bool part = 10 * vecs <= 6 * 64 * groups;     // 60% of them
+  const bool full = 10 * vecs >= 9 * 64 * groups;     // 90%
+  // rounds that the column kernel does not fill (its ordered rounds are 32 rows)
+  const bool brief = R < (ordered && (es < 8 || part) ? 64 : 25) && (!ordered || part || R % 32 != 0);
+  const bool ragged = C % V != 0;  // rows start anywhere: (1000, 200003) f32 sum 147 us by columns, 120 by lanes
+  if (C >= V && items < (uint64_t(1) << 31) &&
+      ((items >= kLaneItems && (narrow || (ordered && brief) || (ragged && full))) ||
+       (items >= 2 * kLaneItems && (brief || (full && (kind != RedKind::kComplexSum || items >= 4 * kLaneItems)))) ||
+       items >= 8 * kLaneItems)) {
+    r.kind = ColRoute::kLanes;
+    return r;
+  }
+  const uint64_t row = C * es;
+  if (row > kSpanRowBytes || (ordered && row == kSpanRowBytes)) return r;
+  const bool contiguous = p.rstride == int64_t(C);
+  if ((C % V != 0 && !contiguous) || R * C < V) return r;
+  const uint64_t round = uint64_t(kSpanBS) * kSpanUnroll * V;  // elements of one round of a whole block
+  uint64_t cw = span_strip(outer, R, C, es, V, round);
+  if (cw == 0) {
+    const uint64_t blocks = outer * groups;  // of the column kernel, before it splits the rows
+    bool span;
+    if (R * C <= round && blocks <= 128)
+      span = true;  // one masked round
+    else if (R <= 24)
+      span = ordered || narrow;
+    else if (blocks <= 24)
+      span = ordered ? outer > 1 || (R >= 20000 && (narrow || (vecs % 64 != 0 && R * row >= (uint64_t(64) << 20))))
+                     : R >= (kind == RedKind::kComplexSum ? 500 : 1400) || (narrow && outer * R >= 8000);
+    else if (narrow)
+      span = true;
+    else if (R <= 128)
+      span = ordered ? row <= 2048 && blocks <= 512 : row <= 1536 && blocks <= (kind == RedKind::kSum ? 128 : 255);
+    else if (kind == RedKind::kComplexSum)  // (two tiles of 128 to 255 blocks would not fit a stream's workspace)
+      span = row <= 2048 || (blocks >= 128 && blocks < 256);
+    else
+      span = R >= (ordered ? 250 : 500) && blocks >= 64 && blocks <= 512 &&
+             (part || (ordered && row <= 2048 && vecs % 64 != 0));
+    if (!span) return r;
+    cw = C;
+  }
+  const uint32_t period = uint32_t(cw) / gcd32(uint32_t(cw), V);  // lanes of the shortest whole-row step
+  if (period > uint32_t(kSpanBS)) return r;
+  r.cw = uint32_t(cw);
+  r.strips = uint32_t(ceil_div(C, cw));
+  if (outer * r.strips * kSpanBlocks >= (uint64_t(1) << 31)) return r;
+  r.kind = ColRoute::kSpans;
+  r.flat = contiguous && r.strips == 1;
+  // the block size with the fewest idle lanes, no larger than one round of the slice needs
+  uint64_t most = ceil_div(ceil_div(R * cw, uint64_t(V) * kSpanUnroll), 64) * 64;
+  const uint64_t least = ceil_div(period, 64) * 64;
+  if (most < least) most = least;
+  if (most > uint64_t(kSpanBS)) most = kSpanBS;
+  for (uint32_t bs = uint32_t(most); bs >= least && 2 * bs > most; bs -= 64) {
+    const uint32_t n = bs / period * period;
+    if (r.bs == 0 || uint64_t(n) * r.bs > uint64_t(r.lanes) * bs + uint64_t(r.bs) * bs / 50) {
+      r.bs = bs;
+      r.lanes = n;
+    }
+  }
+  r.m = uint32_t(uint64_t(r.lanes) * V / cw);
+  // 256 blocks, one per CU with 8 x 16-byte loads in flight per lane, twice buffered ((1000003, 37) f32
+  // mean 30.8 us, 32.8 with 512 and 36.2 with 1024).  A second launch folds the tiles: not worth it
+  // below 6 rounds
+  const uint64_t chunks = R / (uint64_t(r.m) * kSpanUnroll);
+  uint64_t tiles = ceil_div(kSpanBlocks, outer * r.strips);
+  if (tiles > chunks / 2) tiles = chunks / 2;
+  // the partials (at most 2 * es bytes each) have to fit the 1 MiB workspace of a stream
+  const uint64_t room = (uint64_t(1) << 20) / (p.out_size * 2 * es);
+  if (tiles > room) tiles = room;
+  r.tiles = uint32_t(chunks < 6 || tiles < 1 ? 1 : tiles);
+  return r;
+}
+
+}  // namespace mpy

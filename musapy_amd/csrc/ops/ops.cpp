@@ -8,7 +8,7 @@
 // 181-237 with copy_into 816-916).  Phase B only calls the C kernel ABI; there is no host
 // compute path.  Path selection for reductions differs from the reference (which switches on
 // axis_len thresholds, op_builder.rs:2513-2514): the kernel library reports how many tiles per
-// output a reduction needs to fill the GPU (musapy_reduce_tiles_hint) and the op layer uses the
+// output a reduction needs to fill the GPU (musapy_reduce_tiles_hint_v2) and the op layer uses the
 // single-pass entry point when that is 1, partial + final otherwise.
 #include "ops.hpp"
 
@@ -733,7 +733,8 @@ Array reduction_axis(const Array& a, std::optional<size_t> axis, bool keepdims, 
       return r;
     }
     size_t tiles = axis_len == 0 ? 1
-                                 : musapy_reduce_tiles_hint(c.nd, c.shape, c.strides, c.axis, axis_len, out_size, es);
+                                 : musapy_reduce_tiles_hint_v2(red_op(k), int(ct), c.nd, c.shape, c.strides, c.axis,
+                                                               axis_len, out_size);
     if (tiles <= 1) {
       red_single(k, ct, c, r.data_ptr());
     } else if (red_fused(k, ct, c, r.data_ptr(), tiles, *s)) {

@@ -14,6 +14,7 @@
 #include <optional>
 
 #include "../kernels/plan.hpp"
+#include "../kernels/routes.hpp"
 #include "../ops/dlpack.hpp"
 #include "../ops/ops.hpp"
 #include "../../../include/musapy_hip_runtime.h"
@@ -650,6 +651,20 @@ PYBIND11_MODULE(_core, m) {
     d["rstride"] = p.rstride;
     d["kind"] = p.kind == mpy::kColReduce ? "col" : "row";
     d["tiles"] = musapy_reduce_tiles_hint(int(shape.size()), shape.data(), strides.data(), axis, shape[axis], out, 4);
+    return d;
+  });
+  // the kernel a column reduction takes: elements of `es` bytes; kind 0 sums, 1 complex sums, 2 max / min / arg
+  m.def("_route_columns", [](const Shape& shape, const Strides& strides, int axis, size_t es, int kind) {
+    mpy::ReducePlan p{};
+    size_t out = 1;
+    for (size_t i = 0; i < shape.size(); ++i)
+      if (int(i) != axis) out *= shape[i];
+    mpy::plan_reduce(p, int(shape.size()), shape.data(), strides.data(), axis, shape[axis], out);
+    const mpy::ColRoute r = mpy::col_route(p, es, mpy::RedKind(kind));
+    py::dict d;
+    d["kind"] = r.kind == mpy::ColRoute::kLanes ? "lanes" : r.kind == mpy::ColRoute::kSpans ? "spans" : "columns";
+    d["strips"] = r.strips;
+    d["tiles"] = r.tiles;
     return d;
   });
   m.def("_plan_scan", [](const Shape& shape, const Strides& strides, int axis) {

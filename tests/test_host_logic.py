@@ -154,3 +154,28 @@ def test_import_fails_loudly_without_device():
         pytest.skip("a device is present")
     with pytest.raises(Exception):
         ms.array([1.0, 2.0])
+
+
+# (shape, axis, element bytes, kind) -> kernel; kind 0 sums, 1 complex sums, 2 max / min / arg
+COLUMN_ROUTES = [
+    ([20000, 16, 8], 1, 4, 0, "lanes"), ([1000, 16, 512], 1, 4, 2, "lanes"), ([4000, 100, 300], 1, 4, 0, "lanes"),
+    ([1000, 120003], 0, 4, 0, "columns"), ([1000, 300000], 0, 4, 0, "lanes"),
+    ([256, 500, 512], 1, 4, 2, "columns"), ([4000, 100, 100], 1, 4, 0, "columns"),
+    ([300, 131072], 0, 4, 2, "columns"), ([1000003, 37], 0, 4, 0, "spans"), ([1000003, 37], 0, 8, 2, "spans"),
+    ([131072, 384], 0, 4, 0, "spans"), ([64, 100, 1000], 1, 4, 0, "columns"), ([120, 2000, 1024], 1, 4, 0, "columns"),
+    ([4000, 128], 0, 4, 2, "columns"), ([4000, 128], 0, 4, 0, "spans"), ([8, 600, 128], 1, 8, 1, "spans"),
+    ([8, 600, 128], 1, 8, 0, "columns"), ([8, 4096, 1000], 1, 4, 0, "columns"), ([8192, 8192], 0, 4, 0, "columns"),
+]
+
+
+@pytest.mark.parametrize("shape,axis,es,kind,want", COLUMN_ROUTES, ids=str)
+def test_column_reduction_routes(shape, axis, es, kind, want):
+    strides = [int(np.prod(shape[i + 1:], dtype=np.int64)) for i in range(len(shape))]
+    assert _core._route_columns(shape, strides, axis, es, kind)["kind"] == want
+
+
+def test_column_strips_and_tiles():
+    """Small inputs split by strips while one is at most one and a half rounds long, else by tiles."""
+    assert _core._route_columns([600, 400], [400, 1], 0, 4, 0)["strips"] > 1
+    r = _core._route_columns([3000, 100], [100, 1], 0, 4, 0)
+    assert r["strips"] == 1 and r["tiles"] > 1
