@@ -1769,9 +1769,16 @@ __global__ __launch_bounds__(kRBlock) void k_reduce_short(const S* __restrict__ 
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (Op::kOrdered && k == 0) first[u] = T(x[u].v[0]);
+      if constexpr (rounds_in_type<Op, T>()) {  // as a tree, like the lanes after it
+        A t[VEC];
 #pragma unroll
-      for (int v = 0; v < VEC; ++v)
-        if (kk + v >= k) acc[u] = Op::step(acc[u], T(x[u].v[v]), int64_t(kk + v));
+        for (int v = 0; v < VEC; ++v) t[v] = kk + v >= k ? A(T(x[u].v[v])) : Op::init();
+        acc[u] = Op::comb(acc[u], tree_fold<Op>(t));
+      } else {
+#pragma unroll
+        for (int v = 0; v < VEC; ++v)
+          if (kk + v >= k) acc[u] = Op::step(acc[u], T(x[u].v[v]), int64_t(kk + v));
+      }
     }
   }
 #pragma unroll
@@ -1794,6 +1801,7 @@ template <class Op, class T, int VEC, class S, class O>
 bool launch_short(const S* a, RedOut<O> out, const ReducePlan& p, hipStream_t st) {
   const uint64_t vecs = ceil_div(p.R, uint64_t(VEC));
   if (p.rstride != 1 || p.R < uint64_t(VEC) || vecs > 2 * kWave || p.out_size >= (uint64_t(1) << 31)) return false;
+  if (std::is_same_v<S, T> && !short_rows_pay(p.R, vecs, sizeof(typename Op::A), Op::kOrdered)) return false;
   constexpr int U = sizeof(typename Op::A) <= 8 ? 4 : 2;
   const int g = short_group(vecs);
   // below two blocks per CU the rows in flight per group leave the GPU idle: (256, 256) f32 argmax

@@ -144,4 +144,15 @@ inline ColRoute col_route(const ReducePlan& p, size_t es, RedKind kind) {
   return r;
 }
 
+// ---------------------------------------------------------------------------------------------
+// Row lengths that the short-row kernel, whose groups are powers of two, leaves to the kernels with 16
+// lanes or one lane per row: accumulators of more than 8 bytes (two rows in flight per group instead
+// of four) whose rows leave almost half of a group idle.  Its time against theirs, 6M and 40M elements:
+// c64 sums of 33 1.31 and 1.39, of 50 1.0 and 1.05; f64 max of 33 1.12 and 1.19, of 40 1.10 and 1.12, of 5
+// 1.06 and 1.0; f64 sums of 33 and 40 (8 bytes) 0.86 and 0.85, 0.82 and 0.76.
+inline bool short_rows_pay(uint64_t R, uint64_t vecs, size_t acc_bytes, bool ordered) {
+  if (acc_bytes <= 8) return true;
+  return !(ordered && R == 5) && (vecs <= 16 || vecs > (ordered ? 24u : 26u));
+}
+
 }  // namespace mpy

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import musapy_amd as ms
+from tests.conftest import assert_bits_equal
 from tests.test_gpu_reduce import dev
 
 pytestmark = pytest.mark.gpu
@@ -35,3 +36,30 @@ def test_column_sums(dt, shape, axis):
     for got, w in ((ms.sum(X, axis=axis), want), (ms.mean(X, axis=axis), want / shape[axis])):
         err = np.linalg.norm((got.numpy() - w).astype(np.float64)) / np.linalg.norm(w.astype(np.float64))
         assert err <= bound(dt, shape[axis]), err
+
+
+
+def tree(t):
+    """Sums along the last axis, halves first: t[i] + t[i + n / 2] while n > 1."""
+    while t.shape[-1] > 1:
+        h = t.shape[-1] // 2
+        t = t[..., :h] + t[..., h:]
+    return t[..., 0]
+
+
+@pytest.mark.parametrize("cols", [8, 9, 13, 33, 67])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_short_row_sums(dt, cols):
+    """Many short rows: the same bits as a tree over each 16-byte vector and then over the lanes of the row
+    (the vector that the end of a row cuts starts earlier, with zeros for the elements of the one before)."""
+    V = 16 // np.dtype(dt).itemsize
+    vecs = -(-cols // V)
+    lanes = 1 << (vecs - 1).bit_length()
+    rows = 524288 // lanes + 3
+    x = np.random.default_rng(cols).random((rows, cols), dtype=dt) + dt(0.5)
+    t = np.zeros((rows, lanes, V), dt)
+    for v in range(vecs):
+        n = min(V, cols - v * V)
+        t[:, v, V - n:] = x[:, v * V:v * V + n]
+    want = tree(tree(t))
+    assert_bits_equal(ms.sum(dev(x), axis=1).numpy(), want, f"{np.dtype(dt).name} rows of {cols}")

@@ -179,3 +179,10 @@ def test_column_strips_and_tiles():
     assert _core._route_columns([600, 400], [400, 1], 0, 4, 0)["strips"] > 1
     r = _core._route_columns([3000, 100], [100, 1], 0, 4, 0)
     assert r["strips"] == 1 and r["tiles"] > 1
+
+
+def test_short_row_routes():
+    pays = _core._short_rows_pay  # (row length, vectors, accumulator bytes, ordered)
+    assert all(pays(r, -(-r // 4), 4, False) for r in range(4, 513))
+    assert not pays(33, 17, 16, True) and not pays(48, 24, 16, True) and pays(50, 25, 16, True)
+    assert not pays(50, 25, 16, False) and pays(64, 32, 16, False) and not pays(5, 3, 16, True) and pays(6, 3, 16, True)
