@@ -1928,11 +1928,9 @@ void launch_reduce(const T* a, RedOut<T> out, int ndim, const size_t* shape, con
   ra.chunk = chunk;
   ra.nwork = uint64_t(out_size) * tiles;
   const uint64_t seg = chunk < p.R ? chunk : p.R;
-  // a 512-lane block per segment from 16 KB on; max / min / arg from 32 KB, since the few elements
-  // per lane of a shorter one improve the running extreme in nearly every chunk, and each time cost
-  // the search for its index ((16384, 4096) f32 max 65.2 us by blocks, 42.4 by waves; 32 KB rows of
-  // (8192, 8192) 40.1 by blocks, 43.8 by waves)
-  if (seg * sizeof(T) >= (Op::kOrdered ? 32768 : 16384)) {
+  // a 512-lane block per segment from 16 KB on, or a wave for some max / min / arg (see ordered_waves)
+  const bool waves = Op::kOrdered && vec_ok && ordered_waves(seg * sizeof(T), ra.nwork);
+  if (seg * sizeof(T) >= 16384 && !waves) {
     unsigned grid = unsigned(ra.nwork);
     if (vec_ok && aligned && chunk % (uint64_t(kRowBS) * V * 4) == 0 && p.R % chunk == 0)
       k_reduce_row<Op, T, kRowBS, kRowBS, V, 4, WRITE, T, T, true><<<grid, kRowBS, 0, st>>>(a, ra, out);
@@ -1942,7 +1940,7 @@ void launch_reduce(const T* a, RedOut<T> out, int ndim, const size_t* shape, con
       k_reduce_row<Op, T, kRowBS, kRowBS, 1, 8, WRITE><<<grid, kRowBS, 0, st>>>(a, ra, out);
   } else if (seg >= 64) {
     unsigned grid = unsigned(ceil_div(ra.nwork, kRBlock / kWave));
-    if (vec_ok && Op::kOrdered && seg * sizeof(T) >= 16384)
+    if (waves)
       k_reduce_row<Op, T, kRBlock, kWave, V, 4, WRITE><<<grid, kRBlock, 0, st>>>(a, ra, out);
     else if (vec_ok)
       k_reduce_row<Op, T, kRBlock, kWave, V, 2, WRITE><<<grid, kRBlock, 0, st>>>(a, ra, out);

@@ -654,6 +654,7 @@ PYBIND11_MODULE(_core, m) {
     return d;
   });
   m.def("_short_rows_pay", &mpy::short_rows_pay);
+  m.def("_ordered_waves", &mpy::ordered_waves);
   // the kernel a column reduction takes: elements of `es` bytes; kind 0 sums, 1 complex sums, 2 max / min / arg
   m.def("_route_columns", [](const Shape& shape, const Strides& strides, int axis, size_t es, int kind) {
     mpy::ReducePlan p{};

@@ -186,3 +186,10 @@ def test_short_row_routes():
     assert all(pays(r, -(-r // 4), 4, False) for r in range(4, 513))
     assert not pays(33, 17, 16, True) and not pays(48, 24, 16, True) and pays(50, 25, 16, True)
     assert not pays(50, 25, 16, False) and pays(64, 32, 16, False) and not pays(5, 3, 16, True) and pays(6, 3, 16, True)
+
+
+def test_ordered_rows_by_waves():
+    waves = _core._ordered_waves  # (bytes of a row, rows)
+    assert waves(16384, 16384) and waves(16384, 1000) and waves(28000, 1536) and waves(32000, 2048)
+    assert not waves(24000, 500) and not waves(32000, 64) and not waves(32000, 16384)
+    assert not waves(32768, 16384) and not waves(16380, 16384)
