@@ -740,17 +740,17 @@ constexpr int kUnroll = 4;
 // Elements per work item, measured on MI355X (flat kernels, 16M-64M elements):
 //  * binary: one 16-byte load per input (c128 mul at 32 bytes per lane: 5.8 TB/s, at 16: 6.8;
 //    comparisons with wider loads lose: lt f32 at 16 B 6.3 TB/s, 32 B 5.7);
-//  * unary / casts: one 16-byte store per lane, with loads of up to 32 bytes (f32->c64 6.4 vs
-//    5.9 TB/s with 32-byte stores; f64->f32 6.7 with 32-byte loads vs 5.9 with 8-byte stores);
-//    a 1- or 2-byte input is read at least 8 bytes at a time (u8->f32 5.7 vs 5.5 TB/s).
+//  * unary / casts: one 16-byte store per lane, with loads of up to 32 bytes (f32->c64 6.4 vs 5.9 TB/s
+//    with 32-byte stores; f64->f32 6.7 with 32-byte loads vs 5.9 with 8-byte stores).  32 bytes per lane, so
+//    that a 1- or 2-byte input is read 8 bytes at a time, leave the streaming stores 16-byte holes: 16M
+//    i8->f64 49 us, 22 with 16 bytes; u8->f32 22.5 and 12.8; i16->f64 40 and 24.
 template <class T>
 constexpr int vec_of() {
   return sizeof(T) >= 16 ? 1 : (sizeof(T) >= 8 ? 2 : (sizeof(T) == 4 ? 4 : 8));
 }
 template <class TA, class TO>
 constexpr int ew_vec() {
-  constexpr int vo = sizeof(TO) >= 16 ? 1 : int(16 / sizeof(TO));
-  return (sizeof(TA) <= 2 && sizeof(TA) * vo < 8) ? 2 * vo : vo;
+  return sizeof(TO) >= 16 ? 1 : int(16 / sizeof(TO));
 }
 
 inline int mode_of(int64_t s) {
@@ -798,9 +798,10 @@ inline bool at_lines(const Plan& p, int o, const void* ptr) {
 // Output rows off 16 bytes are streamed beside a large input only: next to it streaming measured
 // up to 20% faster (abs of (4097, 7999) slices 54.9 -> 43.7 us), but a lone output, whose lines at
 // the row ends then go out in parts, slower (the outer difference of 8009 and 4003 f64 49.0 -> 59.8).
+// An output written as one run has no such ends.
 template <class TO>
 inline bool out_aligned(const Plan& p, const void* c) {
-  return p.shape[p.ndim - 1] * sizeof(TO) % 16 == 0 && reinterpret_cast<uintptr_t>(c) % 16 == 0;
+  return p.ndim == 1 || (p.shape[p.ndim - 1] * sizeof(TO) % 16 == 0 && reinterpret_cast<uintptr_t>(c) % 16 == 0);
 }
 
 inline unsigned grid_generic(uint64_t n) {
