@@ -18,6 +18,7 @@
 //   generic    64-bit per-element decode, only for shapes beyond the 32-bit limits above.
 #include "kcommon.hpp"
 #include "ew_ops.hpp"
+#include "routes.hpp"
 #include "../../../include/musapy_kernels.h"
 
 namespace mpy {
@@ -767,34 +768,6 @@ inline NdMeta64 make_meta64(const Plan& p) {
   return m;
 }
 
-// distinct elements operand `o` of a plan reads (broadcast dims, stride 0, count once)
-inline uint64_t operand_elems(const Plan& p, int o) {
-  uint64_t n = 1;
-  for (int d = 0; d < p.ndim; ++d)
-    if (p.stride[o][d] != 0) n *= p.shape[d];
-  return n;
-}
-
-// true when every row that operand `o` walks starts on a 128-byte line.  Only then do streaming loads
-// pay: a row that starts inside a line shares its first and last line with its neighbours, and a
-// streamed line is not kept for them.  Measured with rotated buffers, default against streaming
-// loads: x - row of (20011, 3001) 87.6 against 95.1 us in f32 and 210 against 225 in f64, (20000,
-// 3000) f64 196 against 215, neighbours along rows of 4003 f64 90 against 106, but the sum with a
-// transposed (8192, 4096) operand 75.4 against 71.1 us in f32 and 144 against 135 in f64, and exp
-// of that view 102 against 97 us in f64.
-template <class T>
-inline bool at_lines(const Plan& p, int o, const void* ptr) {
-  const int64_t es = int64_t(sizeof(T));
-  uintptr_t q = reinterpret_cast<uintptr_t>(ptr);
-  for (int d = 0; d < p.ndim; ++d) {
-    const int64_t s = p.stride[o][d];
-    if (s == -1) q -= (p.shape[d] - 1) * sizeof(T);  // a flipped row starts at its far end
-    if (s < -1 || s > 1)
-      if (s * es % 128) return false;
-  }
-  return q % 128 == 0;
-}
-
 // Output rows off 16 bytes are streamed beside a large input only: next to it streaming measured
 // up to 20% faster (abs of (4097, 7999) slices 54.9 -> 43.7 us), but a lone output, whose lines at
 // the row ends then go out in parts, slower (the outer difference of 8009 and 4003 f64 49.0 -> 59.8).
@@ -828,7 +801,9 @@ void launch_unary(const TA* a, TO* c, int ndim, const size_t* shape, const ssize
   // the narrower type moves 16 bytes per item, the wider one 16-32 (e.g. f64->f32: 4 elements)
   constexpr int V = ew_vec<TA, TO>();
   const bool big = operand_elems(p, 1) * sizeof(TA) >= kStreamLoadBytes;
-  const bool nt = big && at_lines<TA>(p, 1, a);
+  // off 16 bytes: default 51 against streaming 54 us for abs of (4097, 7999) f32 slices of 8191, 30 against 34
+  // for a run of 16M f32->f64 (abs of one level); on 16 bytes 174 against 168 for (16000, 4096) f64 slices of 4100
+  const bool nt = big && rows_at(p, 1, a, sizeof(TA), 16);
   const bool nts = p.numel * sizeof(TO) >= kStreamStoreBytesUnary && (big || out_aligned<TO>(p, c));
   if (p.ndim == 1 && p.stride[0][0] == 1 && (p.stride[1][0] == 0 || p.stride[1][0] == 1)) {
     In<TA> ia{a, mode_of(p.stride[1][0]), nt};
@@ -860,7 +835,7 @@ void launch_unary(const TA* a, TO* c, int ndim, const size_t* shape, const ssize
         // tiles read across many rows at once: streaming won at 128 MB too (5.1 vs 4.9 TB/s), and with
         // the 1024-lane tiles default loads ran 2-8% slower (f32 X^T 98.1 vs 91.2 us, c128 98.9 vs 91.4);
         // rows off the lines take default loads at any size, see at_lines()
-        ta.nt = at_lines<TA>(p, 1, a);
+        ta.nt = rows_at(p, 1, a, sizeof(TA), kLine);
         for (int d = nd - 2; d >= 0; --d) {
           if (d == P) continue;
           int k = ta.batch.nd++;
@@ -897,10 +872,10 @@ void launch_binary(const T* a, const T* b, TO* c, int ndim, const size_t* shape,
   constexpr int V = vec_of<T>();
   const int nd = p.ndim;
   const bool big = (operand_elems(p, 1) + operand_elems(p, 2)) * sizeof(T) >= kStreamLoadBytes;
-  const bool nt = big && at_lines<T>(p, 1, a) && at_lines<T>(p, 2, b);
+  const LoadPolicy nt = binary_loads(p, a, b, sizeof(T), big);
   const bool nts = p.numel * sizeof(TO) >= kStreamStoreBytes && (big || out_aligned<TO>(p, c));
   if (nd == 1 && (p.stride[1][0] == 0 || p.stride[1][0] == 1) && (p.stride[2][0] == 0 || p.stride[2][0] == 1)) {
-    In<T> ia{a, mode_of(p.stride[1][0]), nt}, ib{b, mode_of(p.stride[2][0]), nt};
+    In<T> ia{a, mode_of(p.stride[1][0]), nt.a}, ib{b, mode_of(p.stride[2][0]), nt.b};
     constexpr uint64_t kTile = uint64_t(kFlatBlockBinary) * V * kFlatUnroll;
     const uint64_t tiles = (p.numel + kTile - 1) / kTile;
     with_store_policy(nts, [&](auto NT) {
@@ -909,11 +884,11 @@ void launch_binary(const T* a, const T* b, TO* c, int ndim, const size_t* shape,
     });
     return;
   }
-  if (launch_binary_transpose<F, T, TO>(a, b, c, p, nt, nts, st, f)) return;
+  if (launch_binary_transpose<F, T, TO>(a, b, c, p, nt.tiles, nts, st, f)) return;
   if (rows_ok(p, V)) {
     const uint32_t L = uint32_t(p.shape[nd - 1]);
     const int64_t sa = p.stride[1][nd - 1], sb = p.stride[2][nd - 1];
-    In<T> ia{a, mode_of(sa), nt}, ib{b, mode_of(sb), nt};
+    In<T> ia{a, mode_of(sa), nt.a}, ib{b, mode_of(sb), nt.b};
     uint32_t gpr = (L + V - 1) / V;
     uint32_t items = uint32_t(p.numel / L) * gpr;
     RowIndexer<3> ix = make_row_indexer<3>(p);
@@ -957,8 +932,7 @@ void launch_binary_mixed(const void* a, const void* b, void* c, int ndim, const 
                                                   : (sizeof(TB) > sizeof(TC) ? sizeof(TB) : sizeof(TC)));
   if (p.ndim == 1 && p.stride[1][0] == 1 && p.stride[2][0] == 1) {
     const uint64_t blocks = (p.numel + uint64_t(kFlatBlockMixed) * V - 1) / (uint64_t(kFlatBlockMixed) * V);
-    const bool nt = p.numel * (sizeof(TA) + sizeof(TB)) >= kStreamLoadBytes && at_lines<TA>(p, 1, a) &&
-                    at_lines<TB>(p, 2, b);
+    const bool nt = p.numel * (sizeof(TA) + sizeof(TB)) >= kStreamLoadBytes;
     const bool nts = p.numel * sizeof(TC) >= kStreamStoreBytes;
     with_store_policy(nts, [&](auto NT) {
       k_binary_flat_mixed<V, NT.value, F, TC, TA, TB><<<dim3(unsigned(blocks)), kFlatBlockMixed, 0, st>>>(

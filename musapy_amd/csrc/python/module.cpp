@@ -653,6 +653,15 @@ PYBIND11_MODULE(_core, m) {
     d["tiles"] = musapy_reduce_tiles_hint(int(shape.size()), shape.data(), strides.data(), axis, shape[axis], out, 4);
     return d;
   });
+  // the load policy of a large binary op whose operands of `es` bytes start at the addresses a and b
+  m.def("_binary_loads", [](const Shape& shape, const std::vector<Strides>& ins, size_t es, uintptr_t a, uintptr_t b) {
+    mpy::Plan p{};
+    std::vector<const ssize_t*> ptrs;
+    for (auto& s : ins) ptrs.push_back(s.data());
+    mpy::plan_elementwise(p, int(shape.size()), shape.data(), int(ins.size()), ptrs.data());
+    const mpy::LoadPolicy l = mpy::binary_loads(p, reinterpret_cast<void*>(a), reinterpret_cast<void*>(b), es, true);
+    return std::vector<bool>{l.a, l.b, l.tiles};
+  });
   m.def("_short_rows_pay", &mpy::short_rows_pay);
   m.def("_ordered_waves", &mpy::ordered_waves);
   // the kernel a column reduction takes: elements of `es` bytes; kind 0 sums, 1 complex sums, 2 max / min / arg

@@ -193,3 +193,21 @@ def test_ordered_rows_by_waves():
     assert waves(16384, 16384) and waves(16384, 1000) and waves(28000, 1536) and waves(32000, 2048)
     assert not waves(24000, 500) and not waves(32000, 64) and not waves(32000, 16384)
     assert not waves(32768, 16384) and not waves(16380, 16384)
+
+
+# which operands of a large f32 binary op stream (first, second, transposed tiles); the operands start at the given
+# addresses, far apart unless `meet`
+@pytest.mark.parametrize("shape,sa,sb,a,b,want", [
+    ((1 << 24,), (1,), (1,), 0, 0, (1, 1, 1)), ((1 << 24,), (1,), (1,), 16, 0, (1, 1, 0)),  # runs
+    ((1 << 24,), (1,), (0,), 4, 0, (1, 0, 0)), ((1 << 24,), (0,), (1,), 0, 0, (0, 1, 1)),  # a scalar
+    ((20000, 4096), (4096, 1), (1, 0), 0, 0, (1, 0, 1)), ((20000, 4003), (4003, 1), (1, 0), 4, 0, (1, 0, 0)),  # a column
+    ((20000, 4096), (4096, 1), (0, 1), 0, 4, (1, 0, 1)), ((20000, 4003), (4003, 1), (0, 1), 0, 0, (0, 0, 0)),  # a row
+    ((20000, 4003), (0, 1), (4003, 1), 0, 0, (0, 0, 0)),
+    ((20000, 4096), (4100, 1), (4100, 1), 0, 0, (1, 1, 0)),  # two slices
+    ((20000, 4003), (4004, 1), (4004, 1), 0, "meet", (0, 0, 0)),  # neighbours in one array
+    ((8192, 4096), (4096, 1), (1, 8192), 0, 0, (1, 1, 1)),  # transposed
+], ids=str)
+def test_binary_loads(shape, sa, sb, a, b, want):
+    base = 1 << 32
+    second = base + 4 if b == "meet" else base * 2 + b
+    assert _core._binary_loads(shape, [sa, sb], 4, base + a, second) == [bool(w) for w in want]
