@@ -496,11 +496,9 @@ bool launch_transpose(const TI* a, TO* c, TransposeArgs ta, uint64_t nb, bool nt
 //  * 8 lanes x 64 rows, 256 lanes: below 4M elements, where the large tile leaves CUs idle ((1000,
 //    700) 4.2 against 6.1 us), and dims of up to 64, half of the large tile ((200000, 37) f32 19.3
 //    against 25.5 us, (16, 200000) 8.4 against 16.3);
-//  * 64 lanes x 32 rows, 512 lanes: L of up to 32 ((200000, 16) f32 10.5 us, small tile 11.2, large
-//    17.6).
-// P and L below 16 keep the row kernels: such tiles would be mostly empty.
-constexpr uint64_t kBinTransposeMin = 16;
-constexpr uint64_t kBinTransposeSmall = uint64_t(4) << 20;
+//  * 64 lanes x 32 rows, 512 lanes: L of up to 32 and a long P ((200000, 16) f32 10.5 us, small tile 11.2,
+//    large 17.6).
+// binary_tile has the lines between them, and to the row kernels.
 struct BinTransposeArgs {
   uint64_t P, L;
   int64_t x_sL;            // stride of x along L (1 along P)
@@ -647,9 +645,8 @@ bool launch_binary_transpose(const T* a, const T* b, TO* c, const Plan& p, bool 
     BinTransposeArgs ta{};
     ta.P = p.shape[P];
     ta.L = p.shape[nd - 1];
-    if (ta.P < kBinTransposeMin || ta.L < kBinTransposeMin || ta.P >= (uint64_t(1) << 32) ||
-        ta.L >= (uint64_t(1) << 32))
-      continue;
+    const BinTile tile = binary_tile(ta.P, ta.L, p.numel, sizeof(T));
+    if (tile == BinTile::kNone || ta.P >= (uint64_t(1) << 32) || ta.L >= (uint64_t(1) << 32)) continue;
     ta.x_sL = xs;
     ta.y_sP = p.stride[3 - o][P];
     ta.y_unit = ys == 1;
@@ -670,8 +667,9 @@ bool launch_binary_transpose(const T* a, const T* b, TO* c, const Plan& p, bool 
     if (!fits) continue;
     const T* x = o == 1 ? a : b;
     const T* y = o == 1 ? b : a;
-    if (ta.L <= 32) return launch_binary_transpose_tiles<F, T, TO, 64, 32, 512, false>(x, y, c, ta, nb, st, f);
-    if (ta.L <= 64 || ta.P <= 64 || p.numel < kBinTransposeSmall)
+    if (tile == BinTile::kTall)
+      return launch_binary_transpose_tiles<F, T, TO, 64, 32, 512, false>(x, y, c, ta, nb, st, f);
+    if (tile == BinTile::kSmall)
       return launch_binary_transpose_tiles<F, T, TO, 8, 64, 256, false>(x, y, c, ta, nb, st, f);
     if (nts) return launch_binary_transpose_tiles<F, T, TO, 32, 128, 1024, true>(x, y, c, ta, nb, st, f);
     return launch_binary_transpose_tiles<F, T, TO, 32, 128, 1024, false>(x, y, c, ta, nb, st, f);

@@ -227,4 +227,29 @@ inline LoadPolicy binary_loads(const Plan& p, const void* a, const void* b, size
   return LoadPolicy{one && !shared, two && !shared, !off_a && !off_b};
 }
 
+// ---------------------------------------------------------------------------------------------
+// The tile of a binary op whose transposed operand is P x L per matrix (elementwise.hip), or none: the
+// row kernels gather the operand from the caches.  P and L below 16 would leave a tile mostly empty.
+// With L of up to 32 even the tall tile is mostly empty when P is short too, and the row kernels win once
+// they fill the GPU.  Sums by rows, tall and small tiles (us):
+//  * below 4 to 12 MB any tile beats the rows: (750, 20, 20) f32 9.0, 5.2 and 3.9; in 16-byte elements
+//    (938, 20, 16) 8.0, 5.7 and 7.1, (625, 20, 24) 7.9, 5.9 and 5.8;
+//  * up to 64 MB the tall tile needs a long P ((4500, 100, 20) f32 35.1 by rows, 29.6 tall; f64 40.7 and 44.6,
+//    so 8-byte elements only up to 48 MB), the small one 32 rows ((8789, 32, 32) f32 34.6, 23.6 small);
+//  * beyond, and from 10 MB in 16 bytes, the rows win ((78125, 16, 16) f32 46, 220 and 92; (12500, 100, 16) 47
+//    and 65 tall) or are level, but for 4-byte matrices that fill a good part of a tall tile: (4883, 128, 32)
+//    51.9 and 44.0, (300, 5000, 17) 101 and 66.
+enum class BinTile { kNone, kTall, kSmall, kLarge };
+inline BinTile binary_tile(uint64_t P, uint64_t L, uint64_t numel, size_t es) {
+  if (P < 16 || L < 16) return BinTile::kNone;
+  if (L > 32) return L <= 64 || P <= 64 || numel < (uint64_t(4) << 20) ? BinTile::kSmall : BinTile::kLarge;
+  const uint64_t mb = numel * es >> 20;
+  if (es >= 16) return mb >= 10 ? BinTile::kNone : L <= 20 ? BinTile::kTall : BinTile::kSmall;
+  const bool tall = P >= (es == 4 ? 100 : 64);
+  if (mb < (tall ? 4 : P * L < 1024 ? 10 : 12)) return BinTile::kSmall;
+  if (mb >= 64) return es == 4 && L > 16 && P * L >= 3072 ? BinTile::kTall : BinTile::kNone;
+  if (tall && (es == 4 || mb < 48)) return BinTile::kTall;
+  return L >= 30 && P >= (es == 4 ? 24 : 32) ? BinTile::kSmall : BinTile::kNone;
+}
+
 }  // namespace mpy

@@ -662,6 +662,10 @@ PYBIND11_MODULE(_core, m) {
     const mpy::LoadPolicy l = mpy::binary_loads(p, reinterpret_cast<void*>(a), reinterpret_cast<void*>(b), es, true);
     return std::vector<bool>{l.a, l.b, l.tiles};
   });
+  m.def("_binary_tile", [](uint64_t P, uint64_t L, uint64_t numel, size_t es) {
+    const char* names[] = {"none", "tall", "small", "large"};
+    return names[int(mpy::binary_tile(P, L, numel, es))];
+  });
   m.def("_short_rows_pay", &mpy::short_rows_pay);
   m.def("_ordered_waves", &mpy::ordered_waves);
   // the kernel a column reduction takes: elements of `es` bytes; kind 0 sums, 1 complex sums, 2 max / min / arg

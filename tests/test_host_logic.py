@@ -211,3 +211,16 @@ def test_binary_loads(shape, sa, sb, a, b, want):
     base = 1 << 32
     second = base + 4 if b == "meet" else base * 2 + b
     assert _core._binary_loads(shape, [sa, sb], 4, base + a, second) == [bool(w) for w in want]
+
+
+# (P, L, elements of the output, element bytes) -> tile of a binary op with a transposed operand
+@pytest.mark.parametrize("args,want", [
+    ((16, 16, 20000000, 4), "none"), ((32, 32, 20000000, 4), "none"), ((32, 16, 30720000, 8), "none"),
+    ((100, 16, 20000000, 4), "none"), ((128, 32, 20000000, 4), "tall"), ((5000, 17, 25500000, 4), "tall"),
+    ((16, 16, 300000, 4), "small"), ((32, 32, 9000000, 4), "small"), ((100, 20, 9000000, 4), "tall"),
+    ((100, 20, 9000000, 8), "none"), ((100, 20, 2000000, 8), "tall"), ((20, 20, 4000000, 16), "none"),
+    ((20, 16, 300000, 16), "tall"), ((24, 32, 300000, 16), "small"), ((15, 4000, 60000, 4), "none"),
+    ((64, 64, 20480000, 4), "small"), ((6000, 5000, 30000000, 4), "large"), ((1000, 700, 700000, 4), "small"),
+], ids=str)
+def test_binary_transpose_tiles(args, want):
+    assert _core._binary_tile(*args) == want
