@@ -252,4 +252,96 @@ inline BinTile binary_tile(uint64_t P, uint64_t L, uint64_t numel, size_t es) {
   return L >= 30 && P >= (es == 4 ? 24 : 32) ? BinTile::kSmall : BinTile::kNone;
 }
 
+// ---------------------------------------------------------------------------------------------
+// How a scan of a strided axis with unit-stride columns runs (scan.hip).
+//
+// Tiles: 16 lanes across (256-byte runs) by 512 lanes of 8 rows, so 256 rows.  The few strips of a
+// narrow array cannot keep the 8 XCDs equally busy under that block numbering, so below 32 strips,
+// where their count is not a multiple of 8, tiles are claimed from a counter instead (their
+// predecessors are then running or finished on whatever XCD), in 512-row tiles of 1024 lanes, which
+// halve the look-backs.  Fewer columns than a 16-byte vector holds take 4 lanes across, one column
+// each.
+//
+// One lane per column keeps the order of the reference, with 32 rows of loads in flight (`depth`):
+// axes of 64 to 384 rows ((300, 20000) f32 26.8 -> 13.9 us; (380, 500) 28.4 -> 14.1), and longer ones
+// of many slices whose rows leave most of a tile's columns idle ((10000, 500, 5) f32 159 us by tiles, 90 by
+// lanes; (50000, 500, 2) 588 and 225; (10000, 1000, 3) f64 350 and 180).  From 512 KB per row of the
+// output on there are lanes enough for longer axes too, with 16 rows in flight ((1000, 131072) f32 184 us, 210 in
+// tiles; (1000, 65536) f64 184 and 209) or, where a row is at most 64 bytes, 32 ((50000, 390, 5) f32 291, 328
+// with 16).
+//
+// kNone, one lane per column with 4 rows in flight, is enough from 1 MB per row on ((1000, 262144) f32 369 us, 411
+// with 16 rows) and from 640 KB on for 8-byte elements and axes below 200 rows ((600, 100000) f64 182 us, 193 with
+// 16; (10, 64, 20000) f32 21.9 and 23.6), and is ahead for some short axes: few columns in f32 ((1000,
+// 64, 2) 13.4 us against 16.2 with 32, (1000, 100, 5) 13.3 and 15.6; in f64 (1000, 100, 2) is 21.0 and 14.7), and
+// rows of 160 bytes and more in f64 ((100, 4096) 9.5 and 10.3).
+constexpr int kColLpc = 16, kColLpcThin = 4, kColBlock = 512, kColBlockClaim = 1024, kColRpl = 8;
+constexpr uint64_t kColClaimGroups = 32;
+constexpr uint64_t kLaneScanRows = 64, kOrderedScanRows = 384;
+struct ColScanRoute {
+  enum : int { kNone = 0, kLane = 1, kTiles = 2 };
+  int kind = kNone;
+  uint32_t cols = 0;                       // lane route: lanes
+  int depth = 0;                           // lane route: rows of loads in flight, 32 or 16
+  bool stream = false;                     // whether a large array may stream
+  uint32_t strips = 0, groups = 0, tiles = 0, per = 0;  // per: groups per tile row of the grid
+  bool claim = false;
+  uint64_t words = 0;                      // tile route: status words (0 for a single tile)
+
+  // Rows that are not whole lines share some with the next row, which other lanes or a later round read, and a
+  // streamed line is not kept for them: lanes along rows of 4 KB and more meet few such lines, tiles of 256-byte
+  // runs from 256 bytes on or with half lines.  (30000, 100, 7) f32 128 us streamed, 82 by default; rows of
+  // 64 bytes, (10000, 390, 8) f64 by lanes, 145 and 134.
+  void lane(const ScanPlan& p, size_t es, int rows_ahead) {
+    const uint64_t row = p.oshape[p.ond - 1] * es;
+    kind = kLane;
+    depth = rows_ahead;
+    stream = row % kLine == 0 || row >= 4096;
+    words = 0;
+  }
+};
+
+// `acc_words`: status words per column and tile, 1 for 4-byte accumulators, else 2
+inline ColScanRoute scan_columns_route(const ScanPlan& p, size_t es, uint64_t acc_words) {
+  ColScanRoute r;
+  const uint64_t VE = 16 / es;
+  const uint64_t C = p.oshape[p.ond - 1];
+  if (p.kind != kColScan || C >= (uint64_t(1) << 31) || p.L >= (uint64_t(1) << 40)) return r;
+  if (p.rows >= (uint64_t(1) << 31)) return r;
+  const uint64_t outer = p.rows / C, row = C * es, kb = p.rows * es >> 10;
+  r.cols = uint32_t(p.rows);
+  if (p.L < kLaneScanRows || kb >= 1024) return r;
+  if (kb >= 512) {
+    if (row <= 64) r.lane(p, es, 32);
+    else if (row < 512 || kb < 640 || (es == 4 && p.L >= 200)) r.lane(p, es, 16);
+    return r;
+  }
+  const bool thin = C < VE;
+  const uint64_t SC = thin ? kColLpcThin : kColLpc * VE;
+  const uint64_t strips = (C + SC - 1) / SC;
+  if (p.L <= kOrderedScanRows) {
+    const bool few = es == 8 ? kb < 48 && row >= 160 && p.L > 64 && p.L <= 112
+                             : row < 32 && p.L <= 256 && kb < (p.L < 100 ? 100 : 48);
+    if (!few) r.lane(p, es, 32);
+    return r;
+  }
+  r.lane(p, es, 32);
+  if (outer >= 5000 && (thin ? p.L <= 512 : strips == 1 && row <= 80)) return r;
+  const uint64_t groups = outer * strips;
+  const bool claim = thin || (groups < kColClaimGroups && groups % 8 != 0);
+  const uint64_t TR = uint64_t(claim ? kColBlockClaim : kColBlock) / (thin ? kColLpcThin : kColLpc) * kColRpl;
+  const uint64_t tiles = (p.L + TR - 1) / TR;
+  const uint64_t per = claim ? groups : (groups + 7) / 8 * 8;
+  if (!grid_fits(per * tiles, claim ? kColBlockClaim : kColBlock)) return r;
+  r.kind = ColScanRoute::kTiles;
+  r.stream = row % 64 == 0 || row >= 256;
+  r.strips = uint32_t(strips);
+  r.groups = uint32_t(groups);
+  r.tiles = uint32_t(tiles);
+  r.per = uint32_t(per);
+  r.claim = claim;
+  r.words = tiles > 1 || claim ? (claim ? 1 : 0) + groups * tiles * SC * acc_words : 0;
+  return r;
+}
+
 }  // namespace mpy

@@ -21,6 +21,7 @@
 // lane and sequential add in exactly the reference CPU order (acc = 0; acc += x[k]).  The tiled
 // paths fix their association by the tile shape, so results are the same bits run to run.
 #include "kcommon.hpp"
+#include "routes.hpp"
 #include "publish.hpp"
 #include "../../../include/musapy_kernels.h"
 
@@ -769,61 +770,9 @@ bool chain_big(const ScanShape& sh) {
   return sh.p.L >= 2 * chain_te<T, kChainBigBlock, kChainBigVpt>();
 }
 
-// How a scan of a strided axis with unit-stride columns runs.
-struct ColScanRoute {
-  enum : int { kNone = 0, kLane = 1, kTiles = 2 };
-  int kind = kNone;
-  uint32_t cols = 0;                       // lane route: lanes
-  uint32_t strips = 0, groups = 0, tiles = 0, per = 0;  // per: groups per tile row of the grid
-  bool claim = false;
-  uint64_t words = 0;                      // tile route: status words (0 for a single tile)
-};
-// 16 lanes across (256-byte runs) by 512 lanes of 8 rows: 256-row tiles.  The few strips of a
-// narrow array cannot keep the 8 XCDs equally busy under the block numbering above, so below 32
-// strips, where their count is not a multiple of 8, tiles are claimed from a counter instead (their
-// predecessors are then running or finished on whatever XCD), in 512-row tiles of 1024 lanes, which
-// halve the look-backs.
-// Fewer columns than a 16-byte vector holds take 4 lanes across, one column each.
-constexpr int kColLpc = 16, kColLpcThin = 4, kColBlock = 512, kColBlockClaim = 1024, kColRpl = 8;
-constexpr uint64_t kColClaimGroups = 32;
-// One lane per column, which keeps the order of the reference, for axes of 64 to 384 rows ((300,
-// 20000) f32 26.8 -> 13.9 us with 32 rows of loads in flight twice over; (380, 500) 28.4 -> 14.1;
-// shorter axes are level with k_scan_seq) and, with 16 rows, for rows of 512 KB and more ((1000,
-// 131072) f32 229 -> 184 us, 210 in tiles; (1000, 65536) f64 203 -> 184, 209 in tiles).  From 1 MB
-// on k_scan_seq has enough lanes to itself: (1000, 262144) f32 369 us, 411 with 16 rows of loads.
-constexpr uint64_t kLaneScanRows = 64, kOrderedScanRows = 384;
-constexpr uint64_t kLaneScanBytes = uint64_t(512) << 10, kSeqScanBytes = uint64_t(1) << 20;
-
 template <class T>
 ColScanRoute col_scan_route(const ScanPlan& p) {
-  ColScanRoute r;
-  constexpr uint64_t VE = 16 / sizeof(T);
-  const uint64_t C = p.oshape[p.ond - 1];
-  if (p.kind != kColScan || C >= (uint64_t(1) << 31) || p.L >= (uint64_t(1) << 40)) return r;
-  const uint64_t outer = p.rows / C;
-  if (p.rows >= (uint64_t(1) << 31)) return r;
-  r.cols = uint32_t(p.rows);
-  const uint64_t row_bytes = p.rows * sizeof(T);
-  if (p.L < kLaneScanRows || row_bytes >= kSeqScanBytes) return r;
-  r.kind = ColScanRoute::kLane;
-  if (p.L <= kOrderedScanRows || row_bytes >= kLaneScanBytes) return r;
-  const bool thin = C < VE;
-  const uint64_t SC = thin ? kColLpcThin : kColLpc * VE;
-  const uint64_t strips = (C + SC - 1) / SC;
-  const uint64_t groups = outer * strips;
-  const bool claim = thin || (groups < kColClaimGroups && groups % 8 != 0);
-  const uint64_t TR = uint64_t(claim ? kColBlockClaim : kColBlock) / (thin ? kColLpcThin : kColLpc) * kColRpl;
-  const uint64_t tiles = (p.L + TR - 1) / TR;
-  const uint64_t per = claim ? groups : (groups + 7) / 8 * 8;
-  if (!grid_fits(per * tiles, claim ? kColBlockClaim : kColBlock)) return r;
-  r.kind = ColScanRoute::kTiles;
-  r.strips = uint32_t(strips);
-  r.groups = uint32_t(groups);
-  r.tiles = uint32_t(tiles);
-  r.per = uint32_t(per);
-  r.claim = claim;
-  r.words = tiles > 1 || claim ? (claim ? 1 : 0) + groups * tiles * SC * (sizeof(typename ScanAcc<T>::A) == 4 ? 1 : 2) : 0;
-  return r;
+  return scan_columns_route(p, sizeof(T), sizeof(typename ScanAcc<T>::A) == 4 ? 1 : 2);
 }
 
 template <class T>
@@ -843,13 +792,13 @@ void launch_scan_columns(const T* a, T* c, const ScanPlan& p, const ColScanRoute
   sa.ls_in = p.ls_in;
   sa.ls_out = p.ls_out;
   const uint64_t bytes = p.rows * p.L * sizeof(T);
-  sa.nt_load = bytes >= kStreamLoadBytes;
-  const bool nts = bytes >= kStreamStoreBytes;
+  sa.nt_load = r.stream && bytes >= kStreamLoadBytes;
+  const bool nts = r.stream && bytes >= kStreamStoreBytes;
   if (r.kind == ColScanRoute::kLane) {
     const unsigned grid = (r.cols + kSBlock - 1) / kSBlock;
     const FastDiv cdiv = make_fastdiv(uint32_t(sa.C));
     with_store_policy(nts, [&](auto NT) {
-      if (p.L <= kOrderedScanRows && p.rows * sizeof(T) < kLaneScanBytes)
+      if (r.depth == 32)
         k_scan_lane<T, 32, NT.value><<<grid, kSBlock, 0, st>>>(a, c, sa, cdiv, r.cols);
       else
         k_scan_lane<T, 16, NT.value><<<grid, kSBlock, 0, st>>>(a, c, sa, cdiv, r.cols);
@@ -1001,9 +950,8 @@ bool run_cumsum(const T* a, T* c, const ScanShape& sh, const ScanScratch& sc, hi
   }
   if (const ColScanRoute r = col_scan_route<T>(p); r.kind != ColScanRoute::kNone) {
     ColScanRoute q = r;
-    // a scratch too small for the status words: one lane per column vector
-    if (q.words != 0 && (sc.lb == nullptr || sc.fault == nullptr || q.words * 8 > sc.lb_bytes))
-      q.kind = ColScanRoute::kLane;
+    // a scratch too small for the status words: one lane per column
+    if (q.words != 0 && (sc.lb == nullptr || sc.fault == nullptr || q.words * 8 > sc.lb_bytes)) q.lane(p, sizeof(T), 32);
     launch_scan_columns<T>(a, c, p, q, sc.lb, sc.fault, sc.clear_fault, st);
     return true;
   }

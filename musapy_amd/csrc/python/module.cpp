@@ -682,6 +682,17 @@ PYBIND11_MODULE(_core, m) {
     d["tiles"] = r.tiles;
     return d;
   });
+  // how a scan of a strided axis runs: elements of `es` bytes
+  m.def("_route_scan", [](const Shape& shape, const Strides& strides, int axis, size_t es) {
+    mpy::ScanPlan p{};
+    mpy::plan_scan(p, int(shape.size()), shape.data(), strides.data(), axis);
+    const mpy::ColScanRoute r = mpy::scan_columns_route(p, es, es == 4 ? 1 : 2);
+    py::dict d;
+    d["kind"] = r.kind == mpy::ColScanRoute::kTiles ? "tiles" : r.kind == mpy::ColScanRoute::kLane ? "lanes" : "none";
+    d["depth"] = r.depth;
+    d["stream"] = r.stream;
+    return d;
+  });
   m.def("_plan_scan", [](const Shape& shape, const Strides& strides, int axis) {
     mpy::ScanPlan p{};
     mpy::plan_scan(p, int(shape.size()), shape.data(), strides.data(), axis);

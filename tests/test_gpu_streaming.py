@@ -48,3 +48,22 @@ def test_transposed_operand_on_lines(dt):
     r, k = 4096, 2048 if dt == np.float64 else 4128  # every row of both operands starts on a line
     a, b = values(dt, (r, k)), values(dt, (k, r))
     assert_bits_equal(ms.sub(dev(a), ms.transpose(dev(b))).numpy(), np.ascontiguousarray(a - b.T), "a - b.T")
+
+
+# (shape, axis): streamed and numbered tiles on lines, and with odd rows; claimed tiles, more than a window of them;
+# one lane per column with 16 rows and, many narrow slices, 32 rows of loads in flight
+@pytest.mark.parametrize("shape,axis", [((8192, 4096), 0), ((8193, 4099), 0), ((12000, 1601), 0), ((450, 131072), 0),
+                                        ((10000, 500, 5), 1), ((30000, 100, 7), 1)], ids=str)
+@pytest.mark.parametrize("dt", [np.int64, np.float32, np.float64])
+def test_column_scans(dt, shape, axis):
+    if dt != np.float32 and shape[-1] > 64:
+        shape = shape[:-1] + (shape[-1] // 2,)
+    x = values(dt, shape)
+    got = ms.cumsum(dev(x), axis=axis).numpy()
+    want = np.cumsum(x, axis, dtype=dt if dt == np.int64 else np.float64 if dt == np.float32 else np.longdouble)
+    if dt == np.int64:
+        assert_bits_equal(got, want, "cumsum")
+        return
+    # any order of n additions is within n * u * sum |x| of the exact sum
+    bound = shape[axis] * np.finfo(dt).eps / 2 * np.cumsum(np.abs(x), axis, dtype=np.float64)
+    assert np.all(np.abs(got - want) <= bound * 1.001)

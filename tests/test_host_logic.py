@@ -224,3 +224,19 @@ def test_binary_loads(shape, sa, sb, a, b, want):
 ], ids=str)
 def test_binary_transpose_tiles(args, want):
     assert _core._binary_tile(*args) == want
+
+
+# (slices, axis, columns), element bytes -> kernel of a cumsum down the axis, rows of loads in flight, streaming
+@pytest.mark.parametrize("shape,es,want", [
+    ((1, 8192, 4096), 4, ("tiles", True)), ((1, 8193, 4099), 4, ("tiles", True)), ((3000, 1000, 24), 4, ("tiles", False)),
+    ((10000, 500, 5), 4, (32, False)), ((50000, 500, 2), 4, (32, False)), ((10000, 1000, 3), 8, (32, False)),
+    ((1000, 500, 5), 4, ("tiles", False)), ((30000, 100, 7), 4, (32, False)), ((5000, 384, 32), 4, (16, True)),
+    ((1, 300, 20000), 4, (32, True)), ((500, 300, 16), 4, (32, False)), ((1, 1000, 131072), 4, (16, True)),
+    ((1, 600, 100000), 8, ("none", False)), ((1, 1000, 262144), 4, ("none", False)), ((1, 63, 4096), 4, ("none", False)),
+    ((1000, 64, 2), 4, ("none", False)), ((10000, 64, 2), 4, ("none", False)), ((100, 100, 64), 8, (32, True)),
+    ((32768, 262144, 2), 4, (32, False)),  # more lanes than a grid dim of tiles holds
+], ids=str)
+def test_column_scan_routes(shape, es, want):
+    o, L, c = shape
+    r = _core._route_scan(list(shape), [L * c, c, 1], 1, es)
+    assert (r["kind"], r["stream"]) == want if isinstance(want[0], str) else (r["kind"], r["depth"], r["stream"]) == ("lanes",) + want
