@@ -3,18 +3,18 @@
 // Drop-in for the reference's kernels/elementwise.mu:577-828 (wrappers) and its nd / flat /
 // vec4 / scalar kernels (elementwise.mu:35-208, 295-394, 451-536).  Instead of one thread per
 // element decoding every dimension with 64-bit div/mod, the wrapper coalesces dimensions on the
-// host (plan.hpp) and picks one of four variants:
+// host (plan.hpp) and picks one of these variants:
 //   flat       every operand contiguous or a broadcast scalar: one 16-byte vector per operand
 //              per lane, many short blocks;
 //   tiles      (binary, long rows) column tiles that walk down the rows: an operand broadcast
 //              along the rows stays in registers, a per-row scalar costs one load per row;
-//   binary transpose  binary ops of one such view and an operand laid out like the output;
 //   rows       output rows of the innermost dim; the outer coordinates of a row are decoded
 //              once with 32-bit magic division, the inner dim is streamed per operand as
 //              vector (stride 1), broadcast (stride 0) or gather (any other stride);
 //   transpose  single-input ops whose input is unit-stride along some other dim (a transposed
 //              or permuted view): 64 x (32*VEC) tiles staged through LDS so that both the read
 //              and the write are 16-byte coalesced accesses;
+//   binary transpose  binary ops of one such view and an operand laid out like the output;
 //   generic    64-bit per-element decode, only for shapes beyond the 32-bit limits above.
 #include "kcommon.hpp"
 #include "ew_ops.hpp"

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import musapy_amd as ms
+from musapy_amd import _core
 from oracle import reference as R
 from tests.conftest import assert_bits_equal
 from tests.test_gpu_reduce import check_reduce, dev
@@ -13,7 +14,7 @@ from tests.test_gpu_reduce import check_reduce, dev
 pytestmark = pytest.mark.gpu
 RNG = np.random.default_rng(4711)
 
-# (shape, axis): what the shape reaches
+# (shape, axis): what the shape reaches; the kernel depends on the type and the op too (ROUTES below pins some)
 SHAPES = [
     ((7, 2), 0), ((2, 3), 0), ((1, 5), 0),                      # a slice of less than one step
     ((50000, 2), 0), ((20000, 3), 0), ((9001, 37), 0),          # short periods, several tiles
@@ -128,9 +129,29 @@ def test_row_views_and_ordered_semantics(kind, dt):
     check_reduce(kind, np.ascontiguousarray(long[:, 1:]), 1, gpu_x=ms.slice(dev(long), [(0, 5, 1), (1, 70003, 1)]))
 
 
+# (shape, axis, kind): kernel, whether its rows are split into tiles, column strips (f32)
+ROUTES = [
+    ((20011, 37), 0, "max", "spans", True, 1), ((20011, 37), 0, "mean", "spans", True, 1),
+    ((40, 600, 37), 1, "argmin", "spans", False, 1), ((300, 700), 0, "max", "spans", False, 44),
+    ((300, 700), 0, "sum", "spans", False, 44), ((12000, 1020), 0, "sum", "spans", True, 1),
+    ((4000, 9, 37), 1, "sum", "lanes", False, 1), ((4000, 9, 37), 1, "argmax", "lanes", False, 1),
+    ((70, 30, 2001), 1, "mean", "lanes", False, 1), ((4097, 96), 0, "max", "columns", False, 1),
+    ((900, 2048), 0, "sum", "columns", False, 1), ((8000, 2048), 0, "argmin", "columns", False, 1),
+]
+
+
+@pytest.mark.parametrize("shape,axis,kind,kernel,tiled,strips", ROUTES, ids=str)
+def test_column_kernels(shape, axis, kind, kernel, tiled, strips):
+    itemsize, order = 4, 0 if kind in ("sum", "mean") else 2
+    steps = [int(np.prod(shape[i + 1:])) for i in range(len(shape))]
+    r = _core._route_columns(list(shape), steps, axis, itemsize, order)
+    assert (r["kind"], r["tiles"] > 1, r["strips"]) == (kernel, tiled, strips)
+    check_reduce(kind, values(kind, np.float32, shape), axis)
+
+
 # ---- cumsum down the columns ----
 SCAN_SHAPES = [
-    ((63, 5), 0), ((64, 3), 0), ((384, 70), 0),                    # sequential, one lane per column
+    ((63, 5), 0), ((64, 3), 0), ((384, 70), 0),                    # one lane per column, in order
     ((385, 64), 0), ((511, 65), 0), ((513, 3), 0),                 # one tile; two; fewer columns than a vector
     ((2049, 1), 0), ((3000, 2), 0), ((2600, 7), 0),                # thin arrays, claimed tiles
     ((1025, 513), 0), ((700, 1030), 0), ((2305, 130), 0),          # strips: a multiple of 8 or not, ragged
