@@ -695,6 +695,27 @@ __device__ inline uint64_t lane_col(const ColArgs& ca, uint32_t cg, int lane) {
   return c0 < ca.C && c0 + VEC > ca.C && ca.C >= VEC ? ca.C - VEC : c0;
 }
 
+// Sums that round in the element's own type (ordered and integer results are exact, and c64 sums run in
+// 64 bits).  The column kernel's 8 waves share the rows of such a sum; a single accumulator for all of
+// them measured an error against 64 bits of 3.6e-7 for f32 sums over 572 rows, where that kernel had
+// 6.7e-8.  So the lane kernel keeps one accumulator per row in flight and joins them as a tree; the
+// span and the column kernel, whose rows are spread over lanes or waves already, add the rows in flight as a
+// tree before they meet the accumulator (accumulators of their own would cost the spans the second block
+// per CU), and the column kernel's waves meet as a tree: f32 sums over the middle of (64, 2048, 384) 4.6e-8
+// against 6.1e-8 with its 4 rows and 8 waves one after the other, 35.7 us both.
+template <class Op, class T>
+constexpr bool rounds_in_type() {
+  return !Op::kOrdered && std::is_same_v<typename Op::A, T>;
+}
+template <class Op, int N>
+__device__ inline typename Op::A tree_fold(typename Op::A (&t)[N]) {
+#pragma unroll
+  for (int h = N / 2; h > 0; h /= 2)
+#pragma unroll
+    for (int u = 0; u < h; ++u) t[u] = Op::comb(t[u], t[u + h]);
+  return t[0];
+}
+
 // One (column group, tile) block of a column reduction: lane `lane` of wave 0 ends with the
 // block's accumulators r[v] of its VEC columns (indices relative to the tile) and first[v], the
 // elements of axis row 0 when the tile starts there.  `part` is the block's LDS for the waves.
@@ -702,6 +723,7 @@ template <class Op, class T, int VEC, int UNROLL, int BS = kRBlock>
 __device__ inline void col_partial(const T* __restrict__ a, const ColArgs& ca, uint32_t t, uint32_t cg,
                                    uint32_t outer, typename Op::A (&part)[BS / kWave - 1][kWave * VEC],
                                    typename Op::A (&acc)[VEC], T (&first)[VEC]) {
+  using A = typename Op::A;
   constexpr int kWaves = BS / kWave;
   const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
   int64_t off[1];
@@ -745,7 +767,14 @@ __device__ inline void col_partial(const T* __restrict__ a, const ColArgs& ca, u
           T xs[UNROLL][1];
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u) xs[u][0] = src[u].v[v];
-          acc[v] = Op::template step_chunk<UNROLL, 1>(acc[v], xs, uint32_t(kk - k0), uint32_t(kWaves));
+          if constexpr (rounds_in_type<Op, T>()) {
+            A p[UNROLL];
+#pragma unroll
+            for (int u = 0; u < UNROLL; ++u) p[u] = xs[u][0];
+            acc[v] = Op::comb(acc[v], tree_fold<Op>(p));
+          } else {
+            acc[v] = Op::template step_chunk<UNROLL, 1>(acc[v], xs, uint32_t(kk - k0), uint32_t(kWaves));
+          }
         }
       };
       if (!Op::kOrdered) {
@@ -797,9 +826,18 @@ __device__ inline void col_partial(const T* __restrict__ a, const ColArgs& ca, u
   __syncthreads();
   if (wv == 0) {
 #pragma unroll
-    for (int v = 0; v < VEC; ++v)
+    for (int v = 0; v < VEC; ++v) {
+      if constexpr (rounds_in_type<Op, T>()) {
+        A p[kWaves];
+        p[0] = acc[v];
 #pragma unroll
-      for (int i = 0; i < kWaves - 1; ++i) acc[v] = Op::comb(acc[v], part[i][lane * VEC + v]);
+        for (int i = 1; i < kWaves; ++i) p[i] = part[i - 1][lane * VEC + v];
+        acc[v] = tree_fold<Op>(p);
+      } else {
+#pragma unroll
+        for (int i = 0; i < kWaves - 1; ++i) acc[v] = Op::comb(acc[v], part[i][lane * VEC + v]);
+      }
+    }
   }
 }
 
@@ -851,24 +889,6 @@ struct SpanArgs {
   int64_t rs;
   bool flat;           // rows are contiguous (rs == C, one strip): a vector may run into the next row
 };
-// Sums that round in the element's own type (ordered and integer results are exact, and c64 sums run in
-// 64 bits).  The column kernel's 8 waves share the rows of such a sum; a single accumulator for all of
-// them measured an error against 64 bits of 3.6e-7 for f32 sums over 572 rows, where that kernel has
-// 6.7e-8.  So the lane kernel keeps one accumulator per row in flight and joins them as a tree, and the
-// span kernel, whose m rows per step are spread over lanes already, adds its 8 rows in flight as a tree
-// before they meet the accumulator (accumulators of their own would cost it the second block per CU).
-template <class Op, class T>
-constexpr bool rounds_in_type() {
-  return !Op::kOrdered && std::is_same_v<typename Op::A, T>;
-}
-template <class Op, int N>
-__device__ inline typename Op::A tree_fold(typename Op::A (&t)[N]) {
-#pragma unroll
-  for (int h = N / 2; h > 0; h /= 2)
-#pragma unroll
-    for (int u = 0; u < h; ++u) t[u] = Op::comb(t[u], t[u + h]);
-  return t[0];
-}
 
 template <class Op, class T, int VEC, int UNROLL, bool FINAL, class S = T, class O = T>
 __global__ __launch_bounds__(kSpanBS) void k_reduce_span(const S* __restrict__ a, SpanArgs sa, RedOut<O> out,

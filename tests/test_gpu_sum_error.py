@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import musapy_amd as ms
+from musapy_amd import _core
 from tests.conftest import assert_bits_equal
 from tests.test_gpu_reduce import dev
 
@@ -37,6 +38,24 @@ def test_column_sums(dt, shape, axis):
         err = np.linalg.norm((got.numpy() - w).astype(np.float64)) / np.linalg.norm(w.astype(np.float64))
         assert err <= bound(dt, shape[axis]), err
 
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_column_kernel_sums(dt):
+    """The column kernel: 8 waves of chains over n / 32 sums of 4 rows, and a tree over the waves.  By the same
+    model u / sqrt(3) * sqrt(8 * 16 * (n / 32)^3 / 3 + 6 * n + 1.75 * n^2) over n, 5.2e-8 in float32 for 400 rows;
+    rows and waves one after the other come to 7.9e-8.  An addition errs by u of the power of two below its result, so
+    the model is itself a bound: about 0.7 of it is expected, 3.8e-8 against 5.7e-8."""
+    n, shape = 400, (80, 400, 1024 if dt == np.float32 else 512)
+    itemsize = np.dtype(dt).itemsize
+    assert _core._route_columns(list(shape), [n * shape[2], shape[2], 1], 1, itemsize, 0)["kind"] == "columns"
+    x = np.random.default_rng(7).random(shape, dtype=dt)
+    x += dt(0.5)
+    want = np.sum(x, axis=1, dtype=np.longdouble)
+    got = ms.sum(dev(x), axis=1).numpy()
+    u = 2.0 ** -24 if dt == np.float32 else 2.0 ** -53
+    model = u / np.sqrt(3) * np.sqrt(8 * 16 * (n / 32) ** 3 / 3 + 6 * n + 1.75 * n ** 2) / n
+    err = np.linalg.norm((got - want).astype(np.float64)) / np.linalg.norm(want.astype(np.float64))
+    assert err <= model, err
 
 
 def tree(t):
