@@ -24,6 +24,8 @@ inline uint32_t gcd32(uint32_t a, uint32_t b) { return b == 0 ? a : gcd32(b, a %
 //    are far apart in memory ((30000, 512) sum 32 -> 14); with many slices of full rows they only cost
 //    ((64, 100, 1000) sum 7.2 -> 14.6, (120, 2000, 1024) 145 -> 183).  Max / min / arg over one slice
 //    keep the column kernel unless the array is long: (4000, 128) 9.0 us, 16.3 by spans.
+//    25 to 63 blocks of the column kernel split into tiles that rarely come to one per CU: (18, 5000, 600)
+//    f32 sum 59 us, 40 by spans, (10, 2100, 700) max 22.4 and 17.7, but (8, 5000, 1000), 256 blocks, 30 and 36.
 //    Inputs of at most 4 MB split by column strips instead of row tiles, which saves the second
 //    launch, if a strip is at most one and a half rounds long: (600, 400) sum 7.3 -> 5.4 us, but (3000,
 //    100) 11.7 by columns, 13.7 by strips and 9.3 by tiles.
@@ -103,7 +105,16 @@ inline ColRoute col_route(const ReducePlan& p, size_t es, RedKind kind) {
       span = true;
     else if (R <= 128)
       span = ordered ? row <= 2048 && blocks <= 512 : row <= 1536 && blocks <= (kind == RedKind::kSum ? 128 : 255);
-    else if (kind == RedKind::kComplexSum)  // (two tiles of 128 to 255 blocks would not fit a stream's workspace)
+    else if (blocks < 64) {
+      // tiles of the column kernel that leave some CUs a second one
+      const bool uneven = row >= 1700 && blocks * ceil_div(uint64_t(256), blocks) > 256;
+      if (ordered)
+        span = part || (R <= 200 ? row <= 2048 : R <= 600 || uneven);
+      else if (kind == RedKind::kComplexSum)
+        span = row <= 2048 || (R >= 500 && uneven);
+      else
+        span = (part && R <= 280) || (R >= 700 && uneven);
+    } else if (kind == RedKind::kComplexSum)  // (two tiles of 128 to 255 blocks would not fit a stream's workspace)
       span = row <= 2048 || (blocks >= 128 && blocks < 256);
     else
       span = R >= (ordered ? 250 : 500) && blocks >= 64 && blocks <= 512 &&

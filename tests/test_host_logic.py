@@ -161,6 +161,8 @@ COLUMN_ROUTES = [
     ([20000, 16, 8], 1, 4, 0, "lanes"), ([1000, 16, 512], 1, 4, 2, "lanes"), ([4000, 100, 300], 1, 4, 0, "lanes"),
     ([1000, 120003], 0, 4, 0, "columns"), ([1000, 300000], 0, 4, 0, "lanes"),
     ([256, 500, 512], 1, 4, 2, "columns"), ([4000, 100, 100], 1, 4, 0, "columns"),
+    ([18, 5000, 600], 1, 4, 0, "spans"), ([8, 5000, 1000], 1, 4, 0, "columns"), ([10, 2100, 700], 1, 4, 2, "spans"),
+    ([52, 263, 54], 1, 8, 2, "spans"), ([14, 500, 432], 1, 4, 0, "columns"), ([12, 2100, 371], 1, 8, 1, "spans"),
     ([300, 131072], 0, 4, 2, "columns"), ([1000003, 37], 0, 4, 0, "spans"), ([1000003, 37], 0, 8, 2, "spans"),
     ([131072, 384], 0, 4, 0, "spans"), ([64, 100, 1000], 1, 4, 0, "columns"), ([120, 2000, 1024], 1, 4, 0, "columns"),
     ([4000, 128], 0, 4, 2, "columns"), ([4000, 128], 0, 4, 0, "spans"), ([8, 600, 128], 1, 8, 1, "spans"),
